@@ -39,7 +39,7 @@
 extern "C" {
 #endif
 
-#define WMX_ABI_VERSION 13
+#define WMX_ABI_VERSION 14
 
 enum {
   WMX_OK = 0,
@@ -483,6 +483,99 @@ typedef struct wmx_feedback_meta_args {
   int32_t use_dummy;          /* 0 or 1 */
 } wmx_feedback_meta_args;
 
+/*
+ * Plans of packed attention calls on the device (the work lists, segment
+ * fields and dS layout that wmx_attn_args takes). Two kinds of input:
+ *   cyclic documents (q_seg != NULL): the int32 metadata of wmx_attn_args over
+ *     (batch, q_len) queries and (batch, k_len) keys at query_stride and
+ *     query_offset. Its packed form is one segment per (row, document): the
+ *     document's queries that see a key, and keys = the leading dummy, then
+ *     the slots from the document's start to its last query's. A
+ *     row that is not run-structured sets WMX_PLAN_REFUSED;
+ *   a packed schedule (q_seg == NULL): query_indices, key_indices, cu_queries
+ *     and cu_keys as in wmx_attn_args, query_stride 1.
+ * Rows that no segment holds follow as segments of their own: runs of queries
+ * without keys, then runs of keys without queries. WMX_PLAN_GENERAL marks
+ * inputs that these kernels do not plan (more than one dummy, key rows other
+ * than slot 0 in two segments, slots that are not consecutive, bounds or
+ * indices out of range).
+ *
+ * wmx_plan_count writes counts (batch + 1, WMX_PLAN_COUNTS) int64, one line
+ * per batch row (packed schedules: the given segments' in line `batch`, with
+ * the number of repeated uses of slot 0 as WMX_PLAN_DUMMIES; counts and
+ * workspace then zero on entry). Unless a flag is set the caller sums the
+ * lines (maxima for the two WMX_PLAN_MAX_), allocates and calls
+ * wmx_plan_fill. The out_ arrays hold WMX_PLAN_QUERIES + IDLE_QUERIES
+ * queries, KEYS + IDLE_KEYS keys and total_segments + 1 bounds; NULL for a
+ * packed schedule without idle rows, which then runs as given. Work lists hold
+ * entries of WMX_UNIT_FIELDS ints, heaviest first; segments of 1 to
+ * fused_rows queries with a key also form f_units, and bq_units / bk_units
+ * are q_units / k_units without them (fused_rows 0: all three NULL).
+ * total_segments < 2^20, key tiles and query tiles of a segment < 2^15.
+ */
+enum {
+  WMX_PLAN_QUERIES = 0,      /* queries of segments */
+  WMX_PLAN_SEGMENTS = 1,
+  WMX_PLAN_KEYS = 2,         /* keys of segments */
+  WMX_PLAN_IDLE_QUERIES = 3, /* queries of no segment, and their runs */
+  WMX_PLAN_QUERY_RUNS = 4,
+  WMX_PLAN_IDLE_KEYS = 5,
+  WMX_PLAN_KEY_RUNS = 6,
+  WMX_PLAN_MAX_QUERIES = 7,  /* largest segment, runs included */
+  WMX_PLAN_MAX_KEYS = 8,
+  WMX_PLAN_Q_UNITS = 9,
+  WMX_PLAN_K_UNITS = 10,
+  WMX_PLAN_F_UNITS = 11,
+  WMX_PLAN_BQ_UNITS = 12,
+  WMX_PLAN_BK_UNITS = 13,
+  WMX_PLAN_DS_ELEMENTS = 14,
+  WMX_PLAN_FLAGS = 15,
+  WMX_PLAN_DUMMIES = 16,     /* leading dummy slots of the row */
+  WMX_PLAN_COUNTS = 17,
+  WMX_PLAN_REFUSED = 1,      /* bits of WMX_PLAN_FLAGS */
+  WMX_PLAN_GENERAL = 2
+};
+
+typedef struct wmx_plan_args {
+  const int32_t* q_seg;
+  const int32_t* k_seg;
+  const int32_t* q_start;
+  const int32_t* k_qend;
+  const int64_t* query_indices;
+  const int64_t* key_indices;
+  const int32_t* cu_queries;
+  const int32_t* cu_keys;
+  void* workspace;            /* wmx_plan_workspace_size bytes, kept from count to fill */
+  int64_t* counts;
+  void* unit_workspace;       /* fill: wmx_plan_unit_workspace_size bytes */
+  int64_t* out_query_indices;
+  int64_t* out_key_indices;
+  int32_t* out_cu_queries;
+  int32_t* out_cu_keys;
+  int32_t* q_units;
+  int32_t* k_units;
+  int32_t* f_units;
+  int32_t* bq_units;
+  int32_t* bk_units;
+  int64_t* ds_offsets;        /* total_segments + 1 */
+  int64_t workspace_bytes;
+  int64_t unit_workspace_bytes;
+  int64_t num_queries;        /* elements of query_indices and key_indices */
+  int64_t num_keys;
+  int32_t num_segments;       /* of the given packed schedule */
+  int32_t batch;
+  int32_t q_len;
+  int32_t k_len;
+  int32_t query_stride;
+  int32_t query_offset;
+  int32_t key_tile;           /* 64 or 128 */
+  int32_t fused_rows;         /* 0 .. 128 */
+  int32_t total_segments;     /* fill: the sizes from the counts */
+  int32_t num_q_units;
+  int32_t num_k_units;
+  int32_t num_f_units;
+} wmx_plan_args;
+
 /* Library identity and struct layout checks for FFI bindings. */
 int wmx_abi_version(void);
 size_t wmx_attn_args_size(void);
@@ -493,6 +586,7 @@ size_t wmx_kv_store_bwd_args_size(void);
 size_t wmx_kv_router_args_size(void);
 size_t wmx_strict_meta_args_size(void);
 size_t wmx_feedback_meta_args_size(void);
+size_t wmx_plan_args_size(void);
 const char* wmx_last_error(void);
 
 /* Forward: o and lse. (see replaced interfaces above) */
@@ -606,6 +700,13 @@ int wmx_strict_meta_fill(const wmx_strict_meta_args* args, void* stream);
  * blocks/_execution/metadata.py:11-55). */
 int64_t wmx_feedback_meta_workspace_size(const wmx_feedback_meta_args* args);
 int wmx_feedback_meta(const wmx_feedback_meta_args* args, void* stream);
+
+/* Plans of packed calls (see wmx_plan_args): no counterpart in the reference,
+ * whose kernels take the metadata as it is. */
+int64_t wmx_plan_workspace_size(const wmx_plan_args* args);
+int64_t wmx_plan_unit_workspace_size(const wmx_plan_args* args);
+int wmx_plan_count(const wmx_plan_args* args, void* stream);
+int wmx_plan_fill(const wmx_plan_args* args, void* stream);
 
 #ifdef __cplusplus
 }

@@ -1,0 +1,118 @@
+"""Plans built on the device (wmx_plan_count / wmx_plan_fill) against the host
+builders on CPU copies of the same tensors, entry for entry: cyclic document
+metadata at strides, residues, dummies, documents and lengths around the
+builders' 1,024-entry chunks, metadata that is not run-structured, and packed
+schedules with padding, short histories and the dummy. The host builders are
+pinned by the oracle on the CPU (tests/test_cyclic_packing.py,
+tests/test_host.py)."""
+
+import importlib
+
+import numpy as np
+import pytest
+import torch
+
+import bench
+from white_matter_amd import prepare_cyclic_attention_metadata, prepare_feedback_metadata, prepare_strict_causal_metadata
+from white_matter_amd import _plans
+
+cyclic = importlib.import_module("white_matter_amd.cyclic_attention")
+strict = importlib.import_module("white_matter_amd.strict_causal_attention")
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _same(device, host, what):
+    assert len(device) == len(host), what
+    for n, (d, h) in enumerate(zip(device, host)):
+        assert d.dtype == h.dtype and d.shape == h.shape and torch.equal(d.cpu(), h), f"{what}: output {n}"
+
+
+def _compare_cyclic(meta, q_len, k_len, stride, offset, what, monkeypatch):
+    meta = [t.to(DEV, torch.int32).contiguous() for t in meta]
+    host = cyclic._cyclic_schedule(*(t.cpu() for t in meta), q_len, k_len, stride, offset)
+    device = cyclic._cyclic_schedule(*meta, q_len, k_len, stride, offset)
+    _same(device, host, what)
+    return int(host[0][0])
+
+
+@pytest.mark.parametrize("dummy", [False, True])
+@pytest.mark.parametrize(("length", "mean", "stride"), [(40, 6, 3), (333, 50, 8), (1024, 200, 2), (2100, 300, 1), (9, 30, 4)])
+def test_cyclic_plans_match_the_host_builder(length, mean, stride, dummy, monkeypatch):
+    docs = bench.geometric_documents(3, length, seed=length + stride, mean=mean, lo=1, hi=length).to(DEV)
+    docs[1] = 0  # a row of one document
+    groups = [torch.arange(r, length, stride, device=DEV) for r in range(stride)]
+    metas = prepare_feedback_metadata(docs, groups, length + int(dummy), use_dummy_token=dummy)
+    for r, meta in enumerate(metas):
+        offset = r if dummy else r - 1
+        status = _compare_cyclic(meta, groups[r].numel(), length + int(dummy), stride, offset, f"residue {r}", monkeypatch)
+        assert status in (1, 2)
+
+
+def test_plans_of_other_metadata_match_the_host_builder(monkeypatch):
+    """Shorter key ranges, two dummies, repeated labels and random metadata:
+    the same plan, or the same refusal."""
+    rng = np.random.default_rng(5)
+    seen = set()
+    for trial in range(60):
+        batch, q_len, stride = int(rng.integers(1, 4)), int(rng.integers(1, 40)), int(rng.integers(1, 4))
+        k_len = stride * (q_len - 1) + 1 + int(rng.integers(0, 20))
+        ids = np.sort(rng.integers(0, 5, (batch, k_len)), 1)
+        kind = trial % 4
+        keys = torch.from_numpy(ids)
+        if kind == 0:
+            keys[:, : int(rng.integers(0, 3))] = -1
+        queries = keys[:, torch.arange(q_len) * stride].clamp_min(0)
+        qstart = torch.searchsorted(keys, queries, right=False)
+        kqend = torch.searchsorted(queries, keys, right=True)
+        kqend[keys < 0] = q_len
+        if kind == 1:  # a label that returns later in the row
+            keys[:, k_len // 2 :] = keys[:, k_len // 2 :] % 2
+        if kind == 2:
+            qstart = qstart + torch.from_numpy(rng.integers(-2, 3, qstart.shape))
+        if kind == 3:
+            kqend = torch.from_numpy(rng.integers(0, q_len + 1, kqend.shape))
+        offset = int(rng.integers(-1, stride))
+        meta = (queries, keys, qstart, kqend)
+        seen.add(_compare_cyclic(meta, q_len, k_len, stride, offset, f"trial {trial}", monkeypatch))
+    assert seen >= {0, 2}
+
+
+def _compare_packed(meta, batch, length, slots, what):
+    given = (meta.query_indices, meta.key_indices, meta.cu_queries, meta.cu_keys)
+    shape = (meta.max_queries, meta.max_keys, batch, length, slots, 4, 2)
+    host = strict._packed_plan(*(t.cpu() for t in given), *shape)
+    device = strict._packed_plan(*given, *shape)
+    for n in (0, *range(1, 11)):
+        if host[n].numel() or device[n].numel():
+            _same([device[n]], [host[n]], f"{what}: output {n}")
+    return host
+
+
+@pytest.mark.parametrize("dummy", [False, True])
+@pytest.mark.parametrize(("length", "mean"), [(17, 4), (300, 40), (1025, 90), (2500, 600)])
+def test_packed_plans_match_the_host_builder(length, mean, dummy):
+    docs = bench.geometric_documents(3, length, seed=length, mean=mean, lo=1, hi=length).to(DEV)
+    docs[1, length // 3 : length // 2] = -1  # padding inside a row
+    docs[2, -3:] = -1
+    meta = prepare_strict_causal_metadata(docs, length, use_dummy_token=dummy)
+    host = _compare_packed(meta, 3, length, length + int(dummy), "documents")
+    assert int(host[0][0]) >= meta.cu_queries.numel() - 1
+    # queries behind a cached prefix: key rows repeat across segments, or sit in a wider pool
+    prefix = length // 2
+    late = prepare_strict_causal_metadata(
+        docs.abs(), length - prefix, query_start=prefix, use_dummy_token=dummy,
+        kv_lengths=torch.tensor([prefix, length, prefix + 3], device=DEV),
+    )
+    _compare_packed(late.with_key_extent(length + 40), 3, length - prefix, length + 40, "cached prefix")
+
+
+def test_plans_take_the_device_path():
+    """The benchmark's forms are planned on the device, not by the host builders."""
+    docs = bench.geometric_documents(2, 512, seed=1).to(DEV)
+    meta = prepare_strict_causal_metadata(docs, 512, use_dummy_token=True)
+    given = (meta.query_indices, meta.key_indices, meta.cu_queries, meta.cu_keys)
+    assert _plans.packed_plan(given, 2, 512, 513, 128) is not None
+    ids = torch.cat((torch.full((2, 1), -1, device=DEV), docs), 1)
+    cyc = prepare_cyclic_attention_metadata(docs[:, ::4].contiguous(), ids)
+    assert _plans.cyclic_plan(tuple(cyc), 128, 513, 4, 0, 64, 96)[0][0] == 2

@@ -19,7 +19,7 @@ import torch
 LIBRARY = Path(__file__).resolve().parent / "lib" / "libwmx_attn.so"
 # the operators registered from C++ (csrc/torch_ops.cpp), linked against LIBRARY
 OPS_LIBRARY = Path(__file__).resolve().parent / "lib" / "libwmx_torch.so"
-ABI_VERSION = 13
+ABI_VERSION = 14
 
 _c_i64_3 = ctypes.c_int64 * 3
 _c_i64_2 = ctypes.c_int64 * 2
@@ -296,6 +296,55 @@ class FeedbackMetaArgs(ctypes.Structure):
     ]
 
 
+# wmx_plan_args counts (WMX_PLAN_*): the columns that the host reads by name
+PLAN_COUNTS = 17
+PLAN_REFUSED, PLAN_GENERAL = 1, 2
+
+
+class PlanArgs(ctypes.Structure):
+    """Mirror of wmx_plan_args."""
+
+    _fields_ = [
+        ("q_seg", _vp),
+        ("k_seg", _vp),
+        ("q_start", _vp),
+        ("k_qend", _vp),
+        ("query_indices", _vp),
+        ("key_indices", _vp),
+        ("cu_queries", _vp),
+        ("cu_keys", _vp),
+        ("workspace", _vp),
+        ("counts", _vp),
+        ("unit_workspace", _vp),
+        ("out_query_indices", _vp),
+        ("out_key_indices", _vp),
+        ("out_cu_queries", _vp),
+        ("out_cu_keys", _vp),
+        ("q_units", _vp),
+        ("k_units", _vp),
+        ("f_units", _vp),
+        ("bq_units", _vp),
+        ("bk_units", _vp),
+        ("ds_offsets", _vp),
+        ("workspace_bytes", ctypes.c_int64),
+        ("unit_workspace_bytes", ctypes.c_int64),
+        ("num_queries", ctypes.c_int64),
+        ("num_keys", ctypes.c_int64),
+        ("num_segments", ctypes.c_int32),
+        ("batch", ctypes.c_int32),
+        ("q_len", ctypes.c_int32),
+        ("k_len", ctypes.c_int32),
+        ("query_stride", ctypes.c_int32),
+        ("query_offset", ctypes.c_int32),
+        ("key_tile", ctypes.c_int32),
+        ("fused_rows", ctypes.c_int32),
+        ("total_segments", ctypes.c_int32),
+        ("num_q_units", ctypes.c_int32),
+        ("num_k_units", ctypes.c_int32),
+        ("num_f_units", ctypes.c_int32),
+    ]
+
+
 EXPORTS = (
     "wmx_abi_version",
     "wmx_attn_args_size",
@@ -331,6 +380,11 @@ EXPORTS = (
     "wmx_feedback_meta_args_size",
     "wmx_feedback_meta_workspace_size",
     "wmx_feedback_meta",
+    "wmx_plan_args_size",
+    "wmx_plan_workspace_size",
+    "wmx_plan_unit_workspace_size",
+    "wmx_plan_count",
+    "wmx_plan_fill",
 )
 
 
@@ -393,6 +447,13 @@ def load() -> ctypes.CDLL:
     lib.wmx_feedback_meta_workspace_size.restype = ctypes.c_int64
     lib.wmx_feedback_meta.argtypes = [ctypes.POINTER(FeedbackMetaArgs), _vp]
     lib.wmx_feedback_meta.restype = ctypes.c_int
+    lib.wmx_plan_args_size.restype = ctypes.c_size_t
+    for name in ("wmx_plan_workspace_size", "wmx_plan_unit_workspace_size"):
+        getattr(lib, name).argtypes = [ctypes.POINTER(PlanArgs)]
+        getattr(lib, name).restype = ctypes.c_int64
+    for name in ("wmx_plan_count", "wmx_plan_fill"):
+        getattr(lib, name).argtypes = [ctypes.POINTER(PlanArgs), _vp]
+        getattr(lib, name).restype = ctypes.c_int
     if lib.wmx_abi_version() != ABI_VERSION:
         raise RuntimeError(f"{path} has ABI {lib.wmx_abi_version()}, expected {ABI_VERSION}")
     if lib.wmx_attn_args_size() != ctypes.sizeof(AttnArgs):
@@ -409,6 +470,8 @@ def load() -> ctypes.CDLL:
         raise RuntimeError("wmx_kv_router_args layout differs between the library and the binding")
     if lib.wmx_feedback_meta_args_size() != ctypes.sizeof(FeedbackMetaArgs):
         raise RuntimeError("wmx_feedback_meta_args layout differs between the library and the binding")
+    if lib.wmx_plan_args_size() != ctypes.sizeof(PlanArgs):
+        raise RuntimeError("wmx_plan_args layout differs between the library and the binding")
     if lib.wmx_strict_meta_args_size() != ctypes.sizeof(StrictMetaArgs):
         raise RuntimeError("wmx_strict_meta_args layout differs between the library and the binding")
     return lib
@@ -550,6 +613,24 @@ def feedback_meta_workspace_size(args: FeedbackMetaArgs) -> int:
 def feedback_meta(args: FeedbackMetaArgs, device: torch.device) -> None:
     lib = load()
     _check(lib, lib.wmx_feedback_meta(ctypes.byref(args), _stream(device)), "wmx_feedback_meta")
+
+
+def plan_workspace_size(args: PlanArgs) -> int:
+    return int(load().wmx_plan_workspace_size(ctypes.byref(args)))
+
+
+def plan_unit_workspace_size(args: PlanArgs) -> int:
+    return int(load().wmx_plan_unit_workspace_size(ctypes.byref(args)))
+
+
+def plan_count(args: PlanArgs, device: torch.device) -> None:
+    lib = load()
+    _check(lib, lib.wmx_plan_count(ctypes.byref(args), _stream(device)), "wmx_plan_count")
+
+
+def plan_fill(args: PlanArgs, device: torch.device) -> None:
+    lib = load()
+    _check(lib, lib.wmx_plan_fill(ctypes.byref(args), _stream(device)), "wmx_plan_fill")
 
 
 def dense_units(args: AttnArgs, units: torch.Tensor, device: torch.device) -> None:

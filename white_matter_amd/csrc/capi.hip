@@ -211,6 +211,44 @@ int check_feedback_meta(const wmx_feedback_meta_args* a) {
   return WMX_OK;
 }
 
+int check_plan(const wmx_plan_args* a, bool fill) {
+  if (!a) return fail(WMX_E_INVALID, "args is NULL");
+  if (a->batch < 1 || a->q_len < 1 || a->k_len < 1) return fail(WMX_E_INVALID, "plans need a nonempty batch, queries and keys");
+  if (a->query_stride < 1) return fail(WMX_E_INVALID, "query_stride must be >= 1");
+  if (a->key_tile != 64 && a->key_tile != 128) return fail(WMX_E_INVALID, "key_tile must be 64 or 128");
+  if (a->fused_rows < 0 || a->fused_rows > 128) return fail(WMX_E_INVALID, "fused_rows must be in [0, 128]");
+  if (a->q_seg) {
+    if (!a->k_seg || !a->q_start || !a->k_qend) return fail(WMX_E_INVALID, "document metadata needs all four arrays");
+  } else {
+    if (!a->query_indices || !a->key_indices || !a->cu_queries || !a->cu_keys)
+      return fail(WMX_E_INVALID, "plans need document metadata or a packed schedule");
+    if (a->num_segments < 1 || a->num_queries < 0 || a->num_keys < 0) return fail(WMX_E_INVALID, "invalid schedule sizes");
+    if (a->query_stride != 1 || a->fused_rows != 0)
+      return fail(WMX_E_INVALID, "packed schedules take query_stride 1 and no fused segments");
+  }
+  if (!a->counts) return fail(WMX_E_INVALID, "counts pointer is NULL");
+  const int64_t need = wmx::plan_workspace_size(*a);
+  if (!a->workspace || a->workspace_bytes < need || !aligned16(a->workspace))
+    return fail(WMX_E_WORKSPACE, "plans need %lld workspace bytes", (long long)need);
+  if (!fill) return WMX_OK;
+  if (a->total_segments < 1 || a->total_segments >= 1 << 20 || a->num_q_units < 0 || a->num_k_units < 0 || a->num_f_units < 0)
+    return fail(WMX_E_INVALID, "invalid plan sizes");
+  const bool own = a->out_query_indices && a->out_key_indices && a->out_cu_queries && a->out_cu_keys;
+  const bool none = !a->out_query_indices && !a->out_key_indices && !a->out_cu_queries && !a->out_cu_keys;
+  if (!own && (a->q_seg || !none || a->total_segments != a->num_segments))
+    return fail(WMX_E_INVALID, "fill needs the covering schedule's arrays");
+  if (!a->ds_offsets || (a->num_q_units && !a->q_units) || (a->num_k_units && !a->k_units) || (a->num_f_units && !a->f_units))
+    return fail(WMX_E_INVALID, "fill needs ds_offsets and the work lists");
+  if (a->fused_rows && (!a->bq_units || !a->bk_units)) return fail(WMX_E_INVALID, "fill needs bq_units and bk_units");
+  for (const void* p : {(const void*)a->q_units, (const void*)a->k_units, (const void*)a->f_units, (const void*)a->bq_units,
+                        (const void*)a->bk_units})
+    if (!aligned16(p)) return fail(WMX_E_INVALID, "work lists must be 16-byte aligned");
+  const int64_t units = wmx::plan_unit_workspace_size(*a);
+  if (!a->unit_workspace || a->unit_workspace_bytes < units || !aligned16(a->unit_workspace))
+    return fail(WMX_E_WORKSPACE, "plans need %lld unit workspace bytes", (long long)units);
+  return WMX_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -446,6 +484,22 @@ int64_t wmx_feedback_meta_workspace_size(const wmx_feedback_meta_args* args) {
 int wmx_feedback_meta(const wmx_feedback_meta_args* a, void* stream) {
   if (const int rc = check_feedback_meta(a)) return rc;
   return launched(wmx::launch_feedback_meta(*a, (hipStream_t)stream));
+}
+
+size_t wmx_plan_args_size(void) { return sizeof(wmx_plan_args); }
+
+int64_t wmx_plan_workspace_size(const wmx_plan_args* a) { return a ? wmx::plan_workspace_size(*a) : 0; }
+
+int64_t wmx_plan_unit_workspace_size(const wmx_plan_args* a) { return a ? wmx::plan_unit_workspace_size(*a) : 0; }
+
+int wmx_plan_count(const wmx_plan_args* a, void* stream) {
+  if (const int rc = check_plan(a, false)) return rc;
+  return launched(wmx::launch_plan_count(*a, (hipStream_t)stream));
+}
+
+int wmx_plan_fill(const wmx_plan_args* a, void* stream) {
+  if (const int rc = check_plan(a, true)) return rc;
+  return launched(wmx::launch_plan_fill(*a, (hipStream_t)stream));
 }
 
 int64_t wmx_decode_workspace_size(const wmx_decode_args* args) {

@@ -72,5 +72,9 @@ int64_t strict_meta_workspace_size(const wmx_strict_meta_args& a);
 int launch_strict_meta(const wmx_strict_meta_args& a, bool fill, hipStream_t stream);
 int64_t feedback_meta_workspace_size(const wmx_feedback_meta_args& a);
 int launch_feedback_meta(const wmx_feedback_meta_args& a, hipStream_t stream);
+int64_t plan_workspace_size(const wmx_plan_args& a);
+int64_t plan_unit_workspace_size(const wmx_plan_args& a);
+int launch_plan_count(const wmx_plan_args& a, hipStream_t stream);
+int launch_plan_fill(const wmx_plan_args& a, hipStream_t stream);
 
 }  // namespace wmx

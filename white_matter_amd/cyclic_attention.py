@@ -29,7 +29,7 @@ from typing import Literal
 
 import torch
 
-from . import _kernels, _native, portable
+from . import _kernels, _native, _plans, portable
 from .metadata import CyclicAttentionMetadata
 
 
@@ -208,6 +208,14 @@ def _cyclic_schedule(
     metadata is not run-structured, or key rows other than the dummy slots
     repeat (the document-mode kernels evaluate the rule per pair)."""
     _kernels.guard_capture("packing cyclic document metadata")
+    from .strict_causal_attention import _FUSED_ROWS, _fused_units, _key_tile, _keys_unique_code, _schedule_flags, _work_units
+
+    meta = (qseg, kseg, qstart, kqend)
+    if qseg.is_cuda and all(t.dtype == torch.int32 and t.is_contiguous() for t in meta):
+        built = _plans.cyclic_plan(meta, q_len, k_len, stride, offset, _key_tile(None, stride), _FUSED_ROWS)
+        if built is not None:
+            facts, tensors = built
+            return [torch.tensor(facts + (0,) * (8 - len(facts)), dtype=torch.int64), *tensors]
     schedule = _build_packed_schedule(qseg, kseg, qstart, kqend, q_len, k_len, stride, offset)
 
     def facts(*values: int) -> torch.Tensor:
@@ -217,8 +225,6 @@ def _cyclic_schedule(
         return [facts(0)]
     if schedule == "empty":
         return [facts(1)]
-    from .strict_causal_attention import _fused_units, _key_tile, _keys_unique_code, _schedule_flags, _work_units
-
     max_q, max_k, flags = _schedule_flags(schedule)
     unique = _keys_unique_code(flags)
     if unique == 0:

@@ -23,7 +23,7 @@ from typing import Literal
 
 import torch
 
-from . import _kernels, _native, portable
+from . import _kernels, _native, _plans, portable
 
 _BACKENDS = ("auto", "reference", "torch_flash", "flash_attention_2")
 
@@ -557,7 +557,7 @@ def _fused_units(
     return lists
 
 
-def _key_tile(metadata: StrictCausalMetadata, stride: int = 1) -> int:
+def _key_tile(metadata: StrictCausalMetadata | None, stride: int = 1) -> int:
     """Keys per dK/dV workgroup for a packed schedule (wmx_attn_args key_tile).
     Strided (cyclic) calls give each key tile few query tiles, so the per-unit
     setup (bounds, K/V rows, first query tiles) dominates: 64-key workgroups,
@@ -799,6 +799,19 @@ def _packed_plan(
     _schedule_gaps) and the work lists q_units, k_units, ds_offsets (see
     _work_units)."""
     _kernels.guard_capture("planning a packed-document schedule")
+    device = query_indices.device
+    given = (query_indices, key_indices, cu_queries, cu_keys)
+    dtypes = (torch.int64, torch.int64, torch.int32, torch.int32)
+    if max_queries == length and all(
+        t.is_cuda and t.is_contiguous() and t.dtype == dtype for t, dtype in zip(given, dtypes)
+    ):
+        built = _plans.packed_plan(given, batch, length, key_slots, _key_tile(None))
+        if built is not None:
+            facts, tensors = built
+            schedule = tensors[:-3] or [torch.empty(0, dtype=torch.int64, device=device) for _ in range(4)]
+            # the covering schedule's segments hold every row: no gaps
+            gaps = [torch.empty(0, dtype=torch.int64, device=device) for _ in range(3)]
+            return [torch.tensor(facts, dtype=torch.int64), *schedule, *gaps, *tensors[-3:]]
     metadata = StrictCausalMetadata(query_indices, key_indices, cu_queries, cu_keys, max_queries, max_keys, key_slots)
     top_q, top_k = _schedule_facts(metadata)[3:5]
     if max_queries != length or top_q >= batch * length or top_k >= batch * key_slots:
@@ -814,7 +827,6 @@ def _packed_plan(
          key_tile],
         dtype=torch.int64,
     )
-    device = query_indices.device
 
     def fresh(t: torch.Tensor) -> torch.Tensor:
         # outputs of an operator may not alias its inputs or each other
