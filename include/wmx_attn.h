@@ -406,6 +406,52 @@ typedef struct wmx_kv_router_args {
 } wmx_kv_router_args;
 
 /*
+ * Backward of the producer (wmx_kv_premix, the router logits, wmx_kv_mix):
+ * the gradients that the reference's autograd gives through `_project`
+ * (modules/kv_pool.py:97-136, modules/routing.py:77-124), with its bf16
+ * roundings of the mixtures' and the logits' gradients and fp32 sums. Inputs
+ * are the forward's; alpha its logits, premixed its premixed rows. The router
+ * reads sources read_start, read_start + read_stride, ...; weight is (C*S,
+ * read_sources * hidden). channels <= 16, C*S <= WMX_KV_ROUTER_MAX_LOGITS,
+ * hidden a multiple of 8 up to 2048. The sums over tokens go through
+ * partial sums in the workspace in a fixed order.
+ */
+#define WMX_KV_MIX_BWD_MAX_CHANNELS 16
+#define WMX_KV_MIX_BWD_MAX_HIDDEN 2048
+
+typedef struct wmx_kv_mix_bwd_args {
+  const void* sources;        /* (B, T, S, hidden), dtype source_dtype, unit stride along hidden */
+  int64_t source_stride[3];   /* element strides [batch, token, source] */
+  const void* premixed[2];    /* bf16 (B*T, S*hidden) contiguous: K side, V side */
+  const void* pre_mix[2];     /* (S, hidden) contiguous, dtype weight_dtype */
+  const void* gain[2];        /* (C, hidden) contiguous, dtype weight_dtype */
+  const void* alpha[2];       /* bf16 (B*T, C*S), rows alpha_stride elements apart */
+  int64_t alpha_stride;
+  const void* weight[2];      /* bf16 (C*S, read_sources * hidden) contiguous */
+  const void* grad[2];        /* bf16 (C, B*T, hidden) contiguous: gradients of the mixtures */
+  void* grad_sources;         /* (B*T, S, hidden) contiguous, dtype source_dtype */
+  void* grad_pre_mix[2];      /* (S, hidden), dtype weight_dtype */
+  void* grad_gain[2];         /* (C, hidden), dtype weight_dtype */
+  void* grad_bias[2];         /* (C*S), dtype grad_weight_dtype */
+  void* grad_weight[2];       /* (C*S, read_sources * hidden) contiguous, dtype grad_weight_dtype */
+  void* workspace;            /* wmx_kv_mix_bwd_workspace_size bytes, 16-byte aligned */
+  int64_t workspace_bytes;
+  int32_t source_dtype;       /* WMX_DTYPE_F32 or WMX_DTYPE_BF16 */
+  int32_t weight_dtype;       /* of pre_mix and gain */
+  int32_t grad_weight_dtype;
+  int32_t batch;
+  int32_t tokens;
+  int32_t num_sources;
+  int32_t hidden;
+  int32_t channels;
+  int32_t read_start;
+  int32_t read_stride;
+  int32_t read_sources;
+  float eps;
+  float mix_eps;
+} wmx_kv_mix_bwd_args;
+
+/*
  * Packed-document schedule builder on the device: the reference's
  * prepare_strict_causal_metadata (ops/strict_causal_attention.py:75-155),
  * whose torch sequence synchronises with the host at every data-dependent
@@ -587,6 +633,7 @@ size_t wmx_kv_router_args_size(void);
 size_t wmx_strict_meta_args_size(void);
 size_t wmx_feedback_meta_args_size(void);
 size_t wmx_plan_args_size(void);
+size_t wmx_kv_mix_bwd_args_size(void);
 const char* wmx_last_error(void);
 
 /* Forward: o and lse. (see replaced interfaces above) */
@@ -700,6 +747,11 @@ int wmx_strict_meta_fill(const wmx_strict_meta_args* args, void* stream);
  * blocks/_execution/metadata.py:11-55). */
 int64_t wmx_feedback_meta_workspace_size(const wmx_feedback_meta_args* args);
 int wmx_feedback_meta(const wmx_feedback_meta_args* args, void* stream);
+
+/* Backward of the producer (see wmx_kv_mix_bwd_args): replaces the autograd of
+ * the reference's eager steps. Outputs are fully overwritten. */
+int64_t wmx_kv_mix_bwd_workspace_size(const wmx_kv_mix_bwd_args* args);
+int wmx_kv_mix_bwd(const wmx_kv_mix_bwd_args* args, void* stream);
 
 /* Plans of packed calls (see wmx_plan_args): no counterpart in the reference,
  * whose kernels take the metadata as it is. */

@@ -281,6 +281,57 @@ def test_producer_training_form_gradients(sources, hidden, channels, stride):
         assert err <= 2e-2, f"{name}: rel-L2 {err:.3e} against float64 autograd of the oracle"
 
 
+@pytest.mark.parametrize(
+    ("batch", "tokens", "sources", "hidden", "channels", "stride", "src_dtype", "weight_dtype"),
+    [
+        (1, 1, 1, 8, 1, 1, torch.float32, torch.float32),  # the smallest of everything
+        (2, 9, 5, 296, 3, 2, torch.float32, torch.bfloat16),  # rows, logits and width off every tile
+        (1, 130, 25, 64, 8, 2, torch.bfloat16, torch.bfloat16),  # past one 128-token block
+        (1, 5, 16, 136, 16, 1, torch.float32, torch.float32),  # the most channels and logits
+        (3, 23, 9, 2048, 4, 2, torch.float32, torch.bfloat16),  # the widest rows
+        (1, 70, 64, 1032, 2, 3, torch.bfloat16, torch.float32),  # just past 1024 elements per thread's first share
+    ],
+)
+def test_producer_backward_kernels(batch, tokens, sources, hidden, channels, stride, src_dtype, weight_dtype):
+    """The backward kernels against float64 autograd of the oracle at the edges
+    of their tiles. The bound: the eager steps they replace round the
+    mixtures', the logits' and the premixed rows' gradients to bf16 too, so the
+    kernels' error may not exceed the eager steps' own by more than a tenth
+    (plus one bf16 rounding of a result, 2^-9)."""
+    stacked, pre_mix, router, gain = _producer_inputs(
+        batch, tokens, sources, hidden, channels, 70 + sources, src_dtype, weight_dtype, stride=stride
+    )
+    flat = [stacked, pre_mix[0], pre_mix[1], *router[0], *router[1], gain[0], gain[1]]
+    leaves = [t.to(DEV).clone().requires_grad_() for t in flat]
+
+    def pairs(t):
+        return (t[1], t[2]), ((t[3], t[4]), (t[5], t[6])), (t[7], t[8])
+
+    assert kv_pool._producer_bwd_fits(sources, hidden, channels)
+    outs = kv_pool.projection_inputs(leaves[0], *pairs(leaves), eps=1e-6, mix_eps=1e-4, router_layer_stride=stride)
+    gen = torch.Generator().manual_seed(3)
+    probe = [torch.randn(o.shape, generator=gen).bfloat16() for o in outs]
+    grads = torch.autograd.grad(outs, leaves, [p.to(DEV) for p in probe])
+    again = torch.autograd.grad(
+        kv_pool.projection_inputs(leaves[0], *pairs(leaves), eps=1e-6, mix_eps=1e-4, router_layer_stride=stride), leaves,
+        [p.to(DEV) for p in probe],
+    )
+    eager = kv_pool._projection_inputs_eager(leaves[0], *pairs(leaves), 1e-6, 1e-4, kv_pool.router_sources(sources, stride))
+    eager_grads = torch.autograd.grad(eager, leaves, [p.to(DEV) for p in probe])
+    wide = [t.detach().cpu().double().requires_grad_() for t in leaves]
+    want = ref.projection_inputs(
+        wide[0], torch.stack(wide[1:3]), ((wide[3], wide[4]), (wide[5], wide[6])), torch.stack(wide[7:9]), 1e-6, 1e-4, stride
+    )
+    exact = torch.autograd.grad(want, wide, torch.stack(probe).double())
+    for n, (g, a, e, r) in enumerate(zip(grads, again, eager_grads, exact)):
+        assert g.dtype == leaves[n].dtype and g.shape == leaves[n].shape
+        assert torch.equal(g, a), f"input {n}: repeats differ"
+        scale = r.norm().clamp_min(1e-30)
+        ours, theirs = ((t.double().cpu() - r).norm() / scale for t in (g, e))
+        print(f"input {n}: kernels {ours:.2e} eager {theirs:.2e}", flush=True)
+        assert ours <= 1.1 * theirs + 2**-9, f"input {n}: rel-L2 {ours:.3e}, the eager steps' {theirs:.3e}"
+
+
 def test_producer_rejects_bad_shapes():
     stacked, pre_mix, router, gain = _producer_inputs(1, 2, 3, 64, 2, 0, torch.float32, torch.float32)
     args = (tuple(pre_mix.to(DEV)), tuple((w.to(DEV), b.to(DEV)) for w, b in router), tuple(gain.to(DEV)))

@@ -296,6 +296,46 @@ class FeedbackMetaArgs(ctypes.Structure):
     ]
 
 
+KV_MIX_BWD_MAX_CHANNELS = 16  # WMX_KV_MIX_BWD_MAX_CHANNELS
+KV_MIX_BWD_MAX_HIDDEN = 2048
+
+
+class KvMixBwdArgs(ctypes.Structure):
+    """Mirror of wmx_kv_mix_bwd_args (index 0 of each pair: the K side, 1: V)."""
+
+    _fields_ = [
+        ("sources", _vp),
+        ("source_stride", ctypes.c_int64 * 3),
+        ("premixed", _vp2),
+        ("pre_mix", _vp2),
+        ("gain", _vp2),
+        ("alpha", _vp2),
+        ("alpha_stride", ctypes.c_int64),
+        ("weight", _vp2),
+        ("grad", _vp2),
+        ("grad_sources", _vp),
+        ("grad_pre_mix", _vp2),
+        ("grad_gain", _vp2),
+        ("grad_bias", _vp2),
+        ("grad_weight", _vp2),
+        ("workspace", _vp),
+        ("workspace_bytes", ctypes.c_int64),
+        ("source_dtype", ctypes.c_int32),
+        ("weight_dtype", ctypes.c_int32),
+        ("grad_weight_dtype", ctypes.c_int32),
+        ("batch", ctypes.c_int32),
+        ("tokens", ctypes.c_int32),
+        ("num_sources", ctypes.c_int32),
+        ("hidden", ctypes.c_int32),
+        ("channels", ctypes.c_int32),
+        ("read_start", ctypes.c_int32),
+        ("read_stride", ctypes.c_int32),
+        ("read_sources", ctypes.c_int32),
+        ("eps", ctypes.c_float),
+        ("mix_eps", ctypes.c_float),
+    ]
+
+
 # wmx_plan_args counts (WMX_PLAN_*): the columns that the host reads by name
 PLAN_COUNTS = 17
 PLAN_REFUSED, PLAN_GENERAL = 1, 2
@@ -380,6 +420,9 @@ EXPORTS = (
     "wmx_feedback_meta_args_size",
     "wmx_feedback_meta_workspace_size",
     "wmx_feedback_meta",
+    "wmx_kv_mix_bwd_args_size",
+    "wmx_kv_mix_bwd_workspace_size",
+    "wmx_kv_mix_bwd",
     "wmx_plan_args_size",
     "wmx_plan_workspace_size",
     "wmx_plan_unit_workspace_size",
@@ -447,6 +490,11 @@ def load() -> ctypes.CDLL:
     lib.wmx_feedback_meta_workspace_size.restype = ctypes.c_int64
     lib.wmx_feedback_meta.argtypes = [ctypes.POINTER(FeedbackMetaArgs), _vp]
     lib.wmx_feedback_meta.restype = ctypes.c_int
+    lib.wmx_kv_mix_bwd_args_size.restype = ctypes.c_size_t
+    lib.wmx_kv_mix_bwd_workspace_size.argtypes = [ctypes.POINTER(KvMixBwdArgs)]
+    lib.wmx_kv_mix_bwd_workspace_size.restype = ctypes.c_int64
+    lib.wmx_kv_mix_bwd.argtypes = [ctypes.POINTER(KvMixBwdArgs), _vp]
+    lib.wmx_kv_mix_bwd.restype = ctypes.c_int
     lib.wmx_plan_args_size.restype = ctypes.c_size_t
     for name in ("wmx_plan_workspace_size", "wmx_plan_unit_workspace_size"):
         getattr(lib, name).argtypes = [ctypes.POINTER(PlanArgs)]
@@ -470,6 +518,8 @@ def load() -> ctypes.CDLL:
         raise RuntimeError("wmx_kv_router_args layout differs between the library and the binding")
     if lib.wmx_feedback_meta_args_size() != ctypes.sizeof(FeedbackMetaArgs):
         raise RuntimeError("wmx_feedback_meta_args layout differs between the library and the binding")
+    if lib.wmx_kv_mix_bwd_args_size() != ctypes.sizeof(KvMixBwdArgs):
+        raise RuntimeError("wmx_kv_mix_bwd_args layout differs between the library and the binding")
     if lib.wmx_plan_args_size() != ctypes.sizeof(PlanArgs):
         raise RuntimeError("wmx_plan_args layout differs between the library and the binding")
     if lib.wmx_strict_meta_args_size() != ctypes.sizeof(StrictMetaArgs):
@@ -613,6 +663,15 @@ def feedback_meta_workspace_size(args: FeedbackMetaArgs) -> int:
 def feedback_meta(args: FeedbackMetaArgs, device: torch.device) -> None:
     lib = load()
     _check(lib, lib.wmx_feedback_meta(ctypes.byref(args), _stream(device)), "wmx_feedback_meta")
+
+
+def kv_mix_bwd_workspace_size(args: KvMixBwdArgs) -> int:
+    return int(load().wmx_kv_mix_bwd_workspace_size(ctypes.byref(args)))
+
+
+def kv_mix_bwd(args: KvMixBwdArgs, device: torch.device) -> None:
+    lib = load()
+    _check(lib, lib.wmx_kv_mix_bwd(ctypes.byref(args), _stream(device)), "wmx_kv_mix_bwd")
 
 
 def plan_workspace_size(args: PlanArgs) -> int:

@@ -368,6 +368,52 @@ int wmx_kv_mix(const wmx_kv_mix_args* a, void* stream) {
   return launched(wmx::launch_kv_mix(*a, (hipStream_t)stream));
 }
 
+static int check_kv_mix_bwd(const wmx_kv_mix_bwd_args* a) {
+  if (!a) return fail(WMX_E_INVALID, "args is NULL");
+  if (a->batch < 1 || a->tokens < 1) return fail(WMX_E_INVALID, "kv mix backward needs tokens");
+  if (a->hidden < 8 || a->hidden % 8 || a->hidden > WMX_KV_MIX_BWD_MAX_HIDDEN)
+    return fail(WMX_E_UNSUPPORTED, "kv mix backward hidden %d is not a multiple of 8 in [8, %d]", a->hidden,
+                WMX_KV_MIX_BWD_MAX_HIDDEN);
+  if (a->channels < 1 || a->channels > WMX_KV_MIX_BWD_MAX_CHANNELS || a->num_sources < 1 ||
+      (int64_t)a->channels * a->num_sources > WMX_KV_ROUTER_MAX_LOGITS)
+    return fail(WMX_E_UNSUPPORTED, "kv mix backward takes up to %d channels and %d logits", WMX_KV_MIX_BWD_MAX_CHANNELS,
+                WMX_KV_ROUTER_MAX_LOGITS);
+  if (a->read_start < 0 || a->read_stride < 1 || a->read_sources < 1 ||
+      a->read_start + (int64_t)(a->read_sources - 1) * a->read_stride >= a->num_sources)
+    return fail(WMX_E_INVALID, "kv mix backward read sources outside the row");
+  for (int dt : {a->source_dtype, a->weight_dtype, a->grad_weight_dtype})
+    if (dt != WMX_DTYPE_F32 && dt != WMX_DTYPE_BF16) return fail(WMX_E_INVALID, "dtype must be WMX_DTYPE_F32 or WMX_DTYPE_BF16");
+  if (!(a->eps >= 0.f) || !(a->mix_eps >= 0.f)) return fail(WMX_E_INVALID, "eps and mix_eps must be >= 0");
+  return WMX_OK;
+}
+
+int64_t wmx_kv_mix_bwd_workspace_size(const wmx_kv_mix_bwd_args* a) {
+  return check_kv_mix_bwd(a) == WMX_OK ? wmx::kv_mix_bwd_workspace_size(*a) : 0;
+}
+
+int wmx_kv_mix_bwd(const wmx_kv_mix_bwd_args* a, void* stream) {
+  if (const int rc = check_kv_mix_bwd(a)) return rc;
+  if (!a->sources || !a->grad_sources) return fail(WMX_E_INVALID, "kv mix backward pointer is NULL");
+  if (!aligned16(a->sources) || !aligned16(a->grad_sources) || !strides_vec8(a->source_stride, 3))
+    return fail(WMX_E_INVALID, "kv mix sources must be 16-byte aligned with strides of multiples of 8 elements");
+  if (a->alpha_stride < (int64_t)a->channels * a->num_sources)
+    return fail(WMX_E_INVALID, "kv mix alpha_stride must cover the C*S logits of a token");
+  for (int side = 0; side < 2; ++side) {
+    for (const void* p : {a->premixed[side], a->pre_mix[side], a->gain[side], a->alpha[side], a->weight[side], a->grad[side],
+                          (const void*)a->grad_pre_mix[side], (const void*)a->grad_gain[side],
+                          (const void*)a->grad_bias[side], (const void*)a->grad_weight[side]})
+      if (!p) return fail(WMX_E_INVALID, "kv mix backward pointer is NULL");
+    for (const void* p : {a->premixed[side], a->pre_mix[side], a->gain[side], a->weight[side], a->grad[side]})
+      if (!aligned16(p)) return fail(WMX_E_INVALID, "kv mix backward operands must be 16-byte aligned");
+  }
+  const int64_t need = wmx::kv_mix_bwd_workspace_size(*a);
+  if (!a->workspace || a->workspace_bytes < need || !aligned16(a->workspace))
+    return fail(WMX_E_WORKSPACE, "kv mix backward needs %lld workspace bytes", (long long)need);
+  return launched(wmx::launch_kv_mix_bwd(*a, (hipStream_t)stream));
+}
+
+size_t wmx_kv_mix_bwd_args_size(void) { return sizeof(wmx_kv_mix_bwd_args); }
+
 static int check_kv_router(const wmx_kv_router_args* a) {
   if (!a) return fail(WMX_E_INVALID, "args is NULL");
   if (a->rows < 0) return fail(WMX_E_INVALID, "negative shape");

@@ -72,6 +72,8 @@ int64_t strict_meta_workspace_size(const wmx_strict_meta_args& a);
 int launch_strict_meta(const wmx_strict_meta_args& a, bool fill, hipStream_t stream);
 int64_t feedback_meta_workspace_size(const wmx_feedback_meta_args& a);
 int launch_feedback_meta(const wmx_feedback_meta_args& a, hipStream_t stream);
+int64_t kv_mix_bwd_workspace_size(const wmx_kv_mix_bwd_args& a);
+int launch_kv_mix_bwd(const wmx_kv_mix_bwd_args& a, hipStream_t stream);
 int64_t plan_workspace_size(const wmx_plan_args& a);
 int64_t plan_unit_workspace_size(const wmx_plan_args& a);
 int launch_plan_count(const wmx_plan_args& a, hipStream_t stream);

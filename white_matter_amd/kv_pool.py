@@ -11,9 +11,10 @@ mix norm and the channel gain cast to bf16 and permuted to (channel, token,
 hidden). `projection_inputs` runs that as three HIP steps: wmx_kv_premix, the
 router logits (wmx_kv_router: a split-K MFMA GEMM, since the library GEMM of
 this shape, few logits over long rows, runs on a few workgroups) and
-wmx_kv_mix. Under autograd the same kernels run forward and the backward
-recomputes the eager steps and differentiates them (the reference's
-selective checkpointing of _project).
+wmx_kv_mix. Under autograd the same kernels run forward, and the backward is
+HIP kernels too (wmx_kv_mix_bwd); sizes that those do not take recompute the
+eager steps and differentiate them (the reference's selective checkpointing of
+_project).
 
 The reference produces a group's keys with an eager sequence
 (src/white_matter/modules/kv_pool.py:163-172 `_apply_k_norm_rope`, the
@@ -196,6 +197,11 @@ def _weights(t: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     return t.to(dtype).contiguous()
 
 
+def _aligned(t: torch.Tensor) -> torch.Tensor:
+    """A contiguous tensor whose rows may be read 16 bytes at a time."""
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def _weight_dtype(*weights: torch.Tensor) -> torch.dtype:
     return torch.bfloat16 if all(t.dtype == torch.bfloat16 for t in weights) else torch.float32
 
@@ -364,19 +370,91 @@ def _projection_inputs_eager(stacked, pre_mix, router, gain, eps, mix_eps, read)
     return out[0], out[1]
 
 
+@torch.library.custom_op("white_matter::kv_producer_bwd", mutates_args=())
+def kv_producer_bwd(
+    stacked: torch.Tensor, pre_k: torch.Tensor, pre_v: torch.Tensor, w_k: torch.Tensor, w_v: torch.Tensor,
+    gain_k: torch.Tensor, gain_v: torch.Tensor, alpha: torch.Tensor, grad_k: torch.Tensor, grad_v: torch.Tensor,
+    eps: float, mix_eps: float, layer_stride: int,
+) -> list[torch.Tensor]:
+    """Gradients of projection_inputs (wmx_kv_mix_bwd) from its inputs, its
+    logits alpha (2, B*T, C*S) and the mixtures' gradients (C, B*T, hidden):
+    stacked, pre_mix K and V, router weight and bias K, weight and bias V, gain
+    K and V, in the inputs' dtypes (biases: the weights')."""
+    batch, tokens, sources, hidden = stacked.shape
+    channels, rows = gain_k.shape[0], batch * tokens
+    device = stacked.device
+    premixed = kv_premix(stacked, pre_k, pre_v, eps)
+    ok = stacked.stride(-1) == 1 and stacked.data_ptr() % 16 == 0 and all(st % 8 == 0 for st in stacked.stride()[:3])
+    x = stacked if ok else _aligned(stacked.contiguous())
+    wdtype = _weight_dtype(pre_k, pre_v, gain_k, gain_v)
+    pre, gains = ([_aligned(_weights(t, wdtype)) for t in pair] for pair in ((pre_k, pre_v), (gain_k, gain_v)))
+    weights, grads = ([_aligned(_weights(t, torch.bfloat16)) for t in pair] for pair in ((w_k, w_v), (grad_k, grad_v)))
+    alpha = alpha.contiguous()
+    read = router_sources(sources, layer_stride)
+    out_dtype = w_k.dtype if w_k.dtype == w_v.dtype and w_k.dtype in _DTYPES else torch.float32
+    d_stacked = torch.empty(stacked.shape, device=device, dtype=x.dtype)
+    d_weight = [torch.empty(w.shape, device=device, dtype=out_dtype) for w in weights]
+    d_pre = [torch.empty(sources, hidden, device=device, dtype=wdtype) for _ in range(2)]
+    d_gain = [torch.empty(channels, hidden, device=device, dtype=wdtype) for _ in range(2)]
+    d_bias = [torch.empty(channels * sources, device=device, dtype=out_dtype) for _ in range(2)]
+    a = _native.KvMixBwdArgs()
+    a.sources, a.source_stride, a.source_dtype = x.data_ptr(), x.stride()[:3], _DTYPES[x.dtype]
+    a.weight_dtype, a.grad_weight_dtype = _DTYPES[wdtype], _DTYPES[out_dtype]
+    a.batch, a.tokens, a.num_sources, a.hidden, a.channels = batch, tokens, sources, hidden, channels
+    a.read_start, a.read_stride, a.read_sources = read.start, read.step, len(read)
+    a.eps, a.mix_eps, a.alpha_stride = float(eps), float(mix_eps), channels * sources
+    a.grad_sources = d_stacked.data_ptr()
+    for side in range(2):
+        a.premixed[side], a.alpha[side] = premixed[side].data_ptr(), alpha[side].data_ptr()
+        a.pre_mix[side], a.gain[side], a.weight[side] = pre[side].data_ptr(), gains[side].data_ptr(), weights[side].data_ptr()
+        a.grad[side] = grads[side].data_ptr()
+        a.grad_pre_mix[side], a.grad_gain[side] = d_pre[side].data_ptr(), d_gain[side].data_ptr()
+        a.grad_bias[side], a.grad_weight[side] = d_bias[side].data_ptr(), d_weight[side].data_ptr()
+    workspace = torch.empty(_native.kv_mix_bwd_workspace_size(a), device=device, dtype=torch.uint8)
+    a.workspace, a.workspace_bytes = workspace.data_ptr(), workspace.numel()
+    _native.kv_mix_bwd(a, device)
+    return [
+        d_stacked, *(d.to(t.dtype) for d, t in zip(d_pre, (pre_k, pre_v))),
+        d_weight[0].to(w_k.dtype), d_bias[0].to(w_k.dtype), d_weight[1].to(w_v.dtype), d_bias[1].to(w_v.dtype),
+        *(d.to(t.dtype) for d, t in zip(d_gain, (gain_k, gain_v))),
+    ]
+
+
+@kv_producer_bwd.register_fake
+def _(stacked, pre_k, pre_v, w_k, w_v, gain_k, gain_v, alpha, grad_k, grad_v, eps, mix_eps, layer_stride):
+    like = [stacked.new_empty(stacked.shape), pre_k.new_empty(pre_k.shape), pre_v.new_empty(pre_v.shape)]
+    for w in (w_k, w_v):
+        like += [w.new_empty(w.shape), w.new_empty(w.shape[0])]
+    return [*like, gain_k.new_empty(gain_k.shape), gain_v.new_empty(gain_v.shape)]
+
+
+def _producer_bwd_fits(sources: int, hidden: int, channels: int) -> bool:
+    """The sizes that wmx_kv_mix_bwd takes (a thread holds a row's share of
+    every channel in registers, and a workgroup the router's columns in LDS);
+    others differentiate the recomputed eager steps."""
+    return (
+        channels <= _native.KV_MIX_BWD_MAX_CHANNELS
+        and channels * sources <= _native.KV_ROUTER_MAX_LOGITS
+        and hidden <= _native.KV_MIX_BWD_MAX_HIDDEN
+    )
+
+
 class _ProjectionInputsFn(torch.autograd.Function):
-    """Training form: the forward runs the HIP kernels; the backward
-    recomputes the reference's eager steps from the saved inputs and
-    differentiates them (the reference trains _project under selective
+    """Training form: HIP kernels forward and backward (wmx_kv_mix_bwd, from
+    the saved inputs and logits). Sizes that the backward kernels do not take
+    recompute the reference's eager steps from the saved inputs and
+    differentiate them (the reference trains _project under selective
     checkpointing with the same recompute)."""
 
     @staticmethod
     def forward(ctx, stacked, pre_k, pre_v, w_k, b_k, w_v, b_v, gain_k, gain_v, eps, mix_eps, stride):
         with torch.no_grad():
-            h_k, h_v = _projection_inputs_hip(
+            h_k, h_v, alphas = _projection_inputs_hip(
                 stacked, (pre_k, pre_v), ((w_k, b_k), (w_v, b_v)), (gain_k, gain_v), eps, mix_eps, stride
             )
-        ctx.save_for_backward(stacked, pre_k, pre_v, w_k, b_k, w_v, b_v, gain_k, gain_v)
+            ctx.on_device = _producer_bwd_fits(*stacked.shape[2:], gain_k.shape[0])
+            kept = (alphas,) if ctx.on_device else ()
+        ctx.save_for_backward(stacked, pre_k, pre_v, w_k, b_k, w_v, b_v, gain_k, gain_v, *kept)
         ctx.config = (eps, mix_eps, stride)
         return h_k, h_v
 
@@ -384,6 +462,14 @@ class _ProjectionInputsFn(torch.autograd.Function):
     def backward(ctx, grad_k, grad_v):
         saved = ctx.saved_tensors
         eps, mix_eps, stride = ctx.config
+        if ctx.on_device:
+            stacked, pre_k, pre_v, w_k, b_k, w_v, b_v, gain_k, gain_v, alpha = saved
+            with torch.no_grad():
+                grads = torch.ops.white_matter.kv_producer_bwd(
+                    stacked, pre_k, pre_v, w_k, w_v, gain_k, gain_v, alpha, grad_k, grad_v, eps, mix_eps, stride
+                )
+                grads = [g.to(t.dtype) if need else None for g, t, need in zip(grads, saved, ctx.needs_input_grad)]
+            return (*grads, None, None, None)
         with torch.enable_grad():
             leaves = [t.detach().requires_grad_(need) for t, need in zip(saved, ctx.needs_input_grad)]
             stacked, pre_k, pre_v, w_k, b_k, w_v, b_v, gain_k, gain_v = leaves
@@ -422,10 +508,10 @@ def projection_inputs(
       alpha = bf16(p[read sources] . W^T + b)         (HIP, wmx_kv_router)
       m = bf16(sum_s alpha[c, s] * p[s])               (HIP, wmx_kv_mix)
       h = bf16(rms_norm(m, mix_eps) * gain[c])
-    Under autograd (any input requiring grad) the forward still runs the HIP
-    kernels and the backward recomputes the reference's eager steps and
-    differentiates them, as the reference trains _project under selective
-    checkpointing. The three HIP steps are the operators white_matter::kv_premix,
+    Under autograd (any input requiring grad) forward and backward run the HIP
+    kernels; sizes beyond the backward's (_producer_bwd_fits) recompute the
+    reference's eager steps and differentiate them, as the reference trains
+    _project under selective checkpointing. The three HIP steps are the operators white_matter::kv_premix,
     white_matter::kv_router and white_matter::kv_mix, so the whole function
     traces under torch.compile. Router widths C*S beyond
     _native.KV_ROUTER_MAX_LOGITS, or S*hidden not a multiple of 64, take the
@@ -439,11 +525,12 @@ def projection_inputs(
             stacked, pre_mix[0], pre_mix[1], w_k, b_k, w_v, b_v, gain[0], gain[1], float(eps), float(mix_eps),
             int(router_layer_stride),
         )
-    return _projection_inputs_hip(stacked, pre_mix, router, gain, eps, mix_eps, router_layer_stride)
+    return _projection_inputs_hip(stacked, pre_mix, router, gain, eps, mix_eps, router_layer_stride)[:2]
 
 
 def _projection_inputs_hip(stacked, pre_mix, router, gain, eps, mix_eps, router_layer_stride):
-    """projection_inputs' forward on the HIP kernels (arguments checked here)."""
+    """projection_inputs' forward on the HIP kernels (arguments checked here):
+    h_K, h_V and both sides' logits (2, B*T, C*S)."""
     if stacked.ndim != 4:
         raise ValueError("stacked must be (B, T, S, hidden)")
     sources, hidden = stacked.shape[2:]
@@ -473,18 +560,16 @@ def _projection_inputs_hip(stacked, pre_mix, router, gain, eps, mix_eps, router_
     gather_ok = router_layer_stride == 1 or hidden % 64 == 0
     if channels * sources <= _native.KV_ROUTER_MAX_LOGITS and (len(read) * hidden) % 64 == 0 and gather_ok:
         (w_k, b_k), (w_v, b_v) = router
-        alphas = torch.ops.white_matter.kv_router(
-            premixed, w_k, b_k, w_v, b_v, hidden, router_layer_stride
-        ).unbind(0)
+        alphas = torch.ops.white_matter.kv_router(premixed, w_k, b_k, w_v, b_v, hidden, router_layer_stride)
     else:
         rows = premixed.shape[1]
-        alphas = [
+        alphas = torch.stack([
             F.linear(
                 premixed[side].view(rows, sources, hidden)[:, read.start :: read.step].reshape(rows, -1),
                 weight.to(torch.bfloat16),
                 bias.to(torch.bfloat16),
             )
             for side, (weight, bias) in enumerate(router)
-        ]
+        ])
     mixed = torch.ops.white_matter.kv_mix(premixed, alphas[0], alphas[1], gain[0], gain[1], float(mix_eps))
-    return mixed[0], mixed[1]
+    return mixed[0], mixed[1], alphas
