@@ -530,6 +530,48 @@ typedef struct wmx_feedback_meta_args {
 } wmx_feedback_meta_args;
 
 /*
+ * The token-local steps between the products of a feedback layer (reference
+ * blocks/decoder_layer.py:51-72, layers/white_matter.py:105-118), with the
+ * reference's fp32 residual policy. Rows are tokens.
+ *   wmx_residual_norm:   x' = x + delta; out = x' (fp32), normed =
+ *     bf16(x' * rsqrt(mean(x'^2) + eps) * weight). delta, out and weight (with
+ *     normed) are optional; out may be x itself.
+ *   wmx_query_norm_rope: per (token, head) row of head_dim elements
+ *     y = bf16(q * rsqrt(mean(q^2) + eps) * weight),
+ *     out = bf16(y * cos + (-y[D/2:], y[:D/2]) * sin).
+ *   wmx_silu_mul:        out = bf16(bf16(gate / (1 + exp(-gate))) * up).
+ */
+typedef struct wmx_residual_norm_args {
+  const float* x;             /* (rows, hidden), rows x_stride elements apart */
+  const void* delta;          /* bf16 (rows, hidden) contiguous, or NULL */
+  const void* weight;         /* (hidden,), dtype weight_dtype, or NULL */
+  float* out;                 /* (rows, hidden), rows out_stride elements apart, or NULL */
+  void* normed;               /* bf16 (rows, hidden) contiguous */
+  int64_t x_stride;
+  int64_t out_stride;
+  int64_t rows;
+  int32_t hidden;             /* a multiple of 8, at most 4096 */
+  int32_t weight_dtype;       /* WMX_DTYPE_F32 or WMX_DTYPE_BF16 */
+  float eps;
+} wmx_residual_norm_args;
+
+typedef struct wmx_query_rope_args {
+  const void* q;              /* bf16 (tokens, heads, head_dim) contiguous */
+  const void* weight;         /* (head_dim,), dtype weight_dtype */
+  const float* cos;           /* fp32 rows of head_dim: token n at
+                                 n / tokens_per_row * rope_stride[0] + n % tokens_per_row * rope_stride[1] */
+  const float* sin;
+  void* out;                  /* bf16 (tokens, heads, head_dim) contiguous */
+  int64_t rope_stride[2];
+  int64_t tokens;
+  int64_t tokens_per_row;
+  int32_t heads;
+  int32_t head_dim;           /* 64, 96 or 128 */
+  int32_t weight_dtype;
+  float eps;
+} wmx_query_rope_args;
+
+/*
  * Plans of packed attention calls on the device (the work lists, segment
  * fields and dS layout that wmx_attn_args takes). Two kinds of input:
  *   cyclic documents (q_seg != NULL): the int32 metadata of wmx_attn_args over
@@ -752,6 +794,11 @@ int wmx_feedback_meta(const wmx_feedback_meta_args* args, void* stream);
  * the reference's eager steps. Outputs are fully overwritten. */
 int64_t wmx_kv_mix_bwd_workspace_size(const wmx_kv_mix_bwd_args* args);
 int wmx_kv_mix_bwd(const wmx_kv_mix_bwd_args* args, void* stream);
+
+/* Steps of a feedback layer (see wmx_residual_norm_args). */
+int wmx_residual_norm(const wmx_residual_norm_args* args, void* stream);
+int wmx_query_norm_rope(const wmx_query_rope_args* args, void* stream);
+int wmx_silu_mul(const void* gate, const void* up, void* out, int64_t n, void* stream);
 
 /* Plans of packed calls (see wmx_plan_args): no counterpart in the reference,
  * whose kernels take the metadata as it is. */

@@ -1,0 +1,94 @@
+"""The layer's fused steps (white_matter::residual_norm, query_norm_rope,
+silu_mul; csrc/layer_ops.hip) against the torch operations they replace, at the
+edges of their row and lane splits, and a model layer through them against the
+same layer through the torch operations.
+
+Bounds: the kernels round where the torch operations do, so results are equal
+except where the fp32 mean's summation order moves a value across a bf16
+rounding boundary: one bf16 step (2^-7 relative at most), on few elements."""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from white_matter_amd.cyclic_pass import FeedbackConfig, FeedbackModel
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+ops = torch.ops.white_matter
+
+
+def _near(got, want, what):
+    g, w = got.float(), want.float()
+    assert g.shape == w.shape and got.dtype == want.dtype, what
+    assert ((g == w) | ((g - w).abs() <= 2**-7 * w.abs() + 1e-6)).all(), what  # (equal infinities differ by nan)
+    assert (g == w).float().mean() > 0.99, what
+
+
+@pytest.mark.parametrize("weight_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize(("shape", "sources"), [((1, 1, 8), 1), ((3, 5, 520), 4), ((2, 33, 1024), 1), ((1, 7, 1032), 3), ((1, 2, 4096), 2)])
+@torch.no_grad()
+def test_residual_norm(shape, sources, weight_dtype):
+    gen = torch.Generator(device=DEV).manual_seed(sum(shape))
+    stacked = torch.randn(*shape[:2], sources, shape[2], generator=gen, device=DEV)
+    x = stacked[:, :, -1]  # rows a multiple of the width apart
+    delta = torch.randn(shape, generator=gen, device=DEV).bfloat16()
+    weight = (1 + 0.1 * torch.randn(shape[2], generator=gen, device=DEV)).to(weight_dtype)
+    out = torch.full((*shape[:2], sources + 1, shape[2]), float("nan"), device=DEV)
+    h = ops.residual_norm(x, delta, out[:, :, 0], weight, 1e-6)
+    want = x + delta.float()
+    assert torch.equal(out[:, :, 0], want) and bool(out[:, :, 1:].isnan().all())
+    _near(h, (F.rms_norm(want, (shape[2],), None, 1e-6) * weight.float()).bfloat16(), "norm of the sum")
+    _near(ops.residual_norm(x, None, None, weight, 1e-6), (F.rms_norm(x, (shape[2],), None, 1e-6) * weight.float()).bfloat16(), "norm")
+    assert ops.residual_norm(x, delta, out[:, :, 0], None, 1e-6).numel() == 0
+    # rows that are not equally spaced, and a misaligned weight
+    odd = torch.randn(shape[0] + 1, shape[1] + 2, shape[2], generator=gen, device=DEV)[1:, 1:-1]
+    shifted = torch.cat((weight[:1], weight))[1:]
+    _near(ops.residual_norm(odd, None, None, shifted, 1e-6), (F.rms_norm(odd, (shape[2],), None, 1e-6) * weight.float()).bfloat16(), "odd rows")
+
+
+@pytest.mark.parametrize(("batch", "length", "heads", "dim"), [(1, 1, 1, 64), (3, 5, 12, 96), (2, 33, 16, 128), (8, 1, 16, 64)])
+@torch.no_grad()
+def test_query_norm_rope(batch, length, heads, dim):
+    gen = torch.Generator(device=DEV).manual_seed(dim + length)
+    q = torch.randn(batch, length, heads * dim, generator=gen, device=DEV).bfloat16()
+    weight = (1 + 0.1 * torch.randn(dim, generator=gen, device=DEV)).bfloat16()
+    angle = torch.rand(batch, length + 2, dim // 2, generator=gen, device=DEV) * 50
+    cos, sin = (torch.cat((t, t), -1)[:, 1:-1] for t in (angle.cos(), angle.sin()))
+    got = ops.query_norm_rope(q, weight, cos, sin, heads, 1e-6)
+    y = F.rms_norm(q.view(batch, length, heads, dim).float(), (dim,), None, 1e-6) * weight.float()
+    y = y.bfloat16().float()
+    rot = torch.cat((-y[..., dim // 2 :], y[..., : dim // 2]), -1)
+    # (the sum of the two products may cancel: one bf16 step of the larger one)
+    want = (y * cos[:, :, None] + rot * sin[:, :, None]).bfloat16()
+    assert got.shape == want.shape and (got == want).float().mean() > 0.99
+    assert ((got.float() - want.float()).abs() <= 2**-7 * (y.abs() + rot.abs())).all()
+
+
+@pytest.mark.parametrize("n", [8, 4096 * 2048 + 8])
+@torch.no_grad()
+def test_silu_mul(n):
+    gen = torch.Generator(device=DEV).manual_seed(n)
+    gate, up = (torch.randn(n, generator=gen, device=DEV).mul(4).bfloat16() for _ in range(2))
+    gate[:3] = torch.tensor([float("inf"), -200.0, 0.0])
+    _near(ops.silu_mul(gate, up), F.silu(gate) * up, "silu")
+
+
+@pytest.mark.parametrize("tokens", [1, 37])
+def test_layer_matches_the_torch_operations(tokens):
+    config = FeedbackConfig(vocab_size=64, hidden_size=136, intermediate_size=264, num_layers=2, num_heads=4, num_kv_heads=2,
+                            head_dim=64, num_kv_channels=2)
+    model = FeedbackModel(config, device=DEV, seed=1)
+    gen = torch.Generator(device=DEV).manual_seed(2)
+    x = torch.randn(2, tokens, 136, generator=gen, device=DEV)
+    rope = model.rope(torch.arange(tokens, device=DEV).expand(2, tokens))
+    attend = lambda q: q.transpose(1, 2) * 0.5  # noqa: E731
+    with torch.no_grad():
+        fused = model.layer(0, x, attend, rope)
+        top, states = model.layers_forward(x, lambda i, q: attend(q), rope)
+        assert torch.equal(states[0], x) and torch.equal(states[1], fused) and torch.equal(states[2], top)
+    with torch.enable_grad():
+        eager = model.layer(0, x.requires_grad_(), attend, rope)  # differentiable: the torch operations
+        eager.sum().backward()
+    # a bf16 rounding moved in the norm reaches the layer's output through two products
+    assert (fused - eager.detach()).norm() <= 2e-3 * (eager.detach() - x.detach()).norm()

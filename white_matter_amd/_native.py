@@ -420,6 +420,9 @@ EXPORTS = (
     "wmx_feedback_meta_args_size",
     "wmx_feedback_meta_workspace_size",
     "wmx_feedback_meta",
+    "wmx_residual_norm",
+    "wmx_query_norm_rope",
+    "wmx_silu_mul",
     "wmx_kv_mix_bwd_args_size",
     "wmx_kv_mix_bwd_workspace_size",
     "wmx_kv_mix_bwd",

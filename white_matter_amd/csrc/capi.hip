@@ -532,6 +532,45 @@ int wmx_feedback_meta(const wmx_feedback_meta_args* a, void* stream) {
   return launched(wmx::launch_feedback_meta(*a, (hipStream_t)stream));
 }
 
+int wmx_residual_norm(const wmx_residual_norm_args* a, void* stream) {
+  if (!a) return fail(WMX_E_INVALID, "args is NULL");
+  if (a->rows < 0 || a->hidden < 8 || a->hidden % 8 || a->hidden > 4096)
+    return fail(WMX_E_UNSUPPORTED, "residual norm hidden %d is not a multiple of 8 in [8, 4096]", a->hidden);
+  if (a->weight_dtype != WMX_DTYPE_F32 && a->weight_dtype != WMX_DTYPE_BF16)
+    return fail(WMX_E_INVALID, "dtype must be WMX_DTYPE_F32 or WMX_DTYPE_BF16");
+  if (!(a->eps >= 0.f)) return fail(WMX_E_INVALID, "eps must be >= 0");
+  if (a->rows == 0) return WMX_OK;
+  if (!a->x || !a->weight != !a->normed || (!a->out && !a->weight)) return fail(WMX_E_INVALID, "residual norm pointer is NULL");
+  if (!aligned16(a->x) || !aligned16(a->delta) || !aligned16(a->weight) || !aligned16(a->out) || !aligned16(a->normed) ||
+      a->x_stride % 4 || a->out_stride % 4)
+    return fail(WMX_E_INVALID, "residual norm operands must be 16-byte aligned rows");
+  return launched(wmx::launch_residual_norm(*a, (hipStream_t)stream));
+}
+
+int wmx_query_norm_rope(const wmx_query_rope_args* a, void* stream) {
+  if (!a) return fail(WMX_E_INVALID, "args is NULL");
+  if (a->head_dim != 64 && a->head_dim != 96 && a->head_dim != 128)
+    return fail(WMX_E_UNSUPPORTED, "head_dim %d is not 64, 96 or 128", a->head_dim);
+  if (a->tokens < 0 || a->heads < 1 || a->tokens_per_row < 1) return fail(WMX_E_INVALID, "negative or zero shape");
+  if (a->weight_dtype != WMX_DTYPE_F32 && a->weight_dtype != WMX_DTYPE_BF16)
+    return fail(WMX_E_INVALID, "dtype must be WMX_DTYPE_F32 or WMX_DTYPE_BF16");
+  if (!(a->eps >= 0.f)) return fail(WMX_E_INVALID, "eps must be >= 0");
+  if (a->tokens == 0) return WMX_OK;
+  if (!a->q || !a->weight || !a->cos || !a->sin || !a->out) return fail(WMX_E_INVALID, "query rope pointer is NULL");
+  if (!aligned16(a->q) || !aligned16(a->weight) || !aligned16(a->cos) || !aligned16(a->sin) || !aligned16(a->out) ||
+      a->rope_stride[0] % 4 || a->rope_stride[1] % 4)
+    return fail(WMX_E_INVALID, "query rope operands must be 16-byte aligned rows");
+  return launched(wmx::launch_query_norm_rope(*a, (hipStream_t)stream));
+}
+
+int wmx_silu_mul(const void* gate, const void* up, void* out, int64_t n, void* stream) {
+  if (n < 0 || n % 8) return fail(WMX_E_INVALID, "silu_mul takes a multiple of 8 elements");
+  if (n == 0) return WMX_OK;
+  if (!gate || !up || !out) return fail(WMX_E_INVALID, "silu_mul pointer is NULL");
+  if (!aligned16(gate) || !aligned16(up) || !aligned16(out)) return fail(WMX_E_INVALID, "silu_mul operands must be 16-byte aligned");
+  return launched(wmx::launch_silu_mul(gate, up, out, n, (hipStream_t)stream));
+}
+
 size_t wmx_plan_args_size(void) { return sizeof(wmx_plan_args); }
 
 int64_t wmx_plan_workspace_size(const wmx_plan_args* a) { return a ? wmx::plan_workspace_size(*a) : 0; }

@@ -920,6 +920,133 @@ void strict_decode_out(const Tensor& out, const Tensor& query, const Tensor& key
               num_splits);
 }
 
+// ------------------------------------------------- layer steps ----
+int32_t float_dtype(const Tensor& t, const char* what) {
+  TORCH_CHECK_TYPE(t.scalar_type() == at::kFloat || t.scalar_type() == at::kBFloat16, what, " must be float32 or bfloat16");
+  return t.scalar_type() == at::kFloat ? WMX_DTYPE_F32 : WMX_DTYPE_BF16;
+}
+
+// The row stride of a (..., hidden) fp32 tensor whose rows are equally spaced.
+bool row_stride(const Tensor& t, int64_t& stride) {
+  if (t.dim() < 1 || t.stride(-1) != 1 || reinterpret_cast<uintptr_t>(t.data_ptr()) % 16) return false;
+  stride = t.size(-1);
+  bool first = true;
+  int64_t next = 0;
+  for (int64_t d = t.dim() - 2; d >= 0; --d) {
+    if (t.size(d) == 1) continue;
+    if (first) stride = next = t.stride(d);
+    else if (t.stride(d) != next) return false;
+    first = false;
+    next *= t.size(d);
+  }
+  return stride % 4 == 0;
+}
+
+// out = x + delta (fp32 rows; delta bf16, optional), and bf16(rms_norm(out) *
+// weight) where a weight is given, else an empty tensor.
+Tensor residual_norm(const Tensor& x, const c10::optional<Tensor>& delta, const c10::optional<Tensor>& out,
+                     const c10::optional<Tensor>& weight, double eps) {
+  TORCH_CHECK_VALUE(x.scalar_type() == at::kFloat && x.dim() >= 1, "residual_norm takes float32 rows");
+  c10::OptionalDeviceGuard guard(x.device());
+  const int64_t hidden = x.size(-1);
+  wmx_residual_norm_args a;
+  std::memset(&a, 0, sizeof(a));
+  Tensor rows = x;
+  if (!row_stride(rows, a.x_stride)) {
+    rows = rows.contiguous().clone();
+    a.x_stride = hidden;
+  }
+  Tensor d, w;
+  a.x = rows.data_ptr<float>();
+  a.rows = hidden ? x.numel() / hidden : 0;
+  a.hidden = (int32_t)hidden;
+  a.eps = (float)eps;
+  if (delta) {
+    TORCH_CHECK_VALUE(delta->sizes() == x.sizes() && delta->scalar_type() == at::kBFloat16 && delta->device() == x.device(),
+                      "delta must be bfloat16 rows like x");
+    d = operand(*delta).contiguous();
+    a.delta = d.data_ptr();
+  }
+  if (out) {
+    TORCH_CHECK_VALUE(out->sizes() == x.sizes() && out->scalar_type() == at::kFloat && out->device() == x.device() &&
+                          row_stride(*out, a.out_stride),
+                      "out must be equally spaced, 16-byte aligned float32 rows like x");
+    a.out = out->data_ptr<float>();
+  }
+  Tensor normed = at::empty(weight ? x.sizes() : c10::IntArrayRef({0}), x.options().dtype(at::kBFloat16));
+  if (weight) {
+    TORCH_CHECK_VALUE(weight->dim() == 1 && weight->size(0) == hidden && weight->device() == x.device(),
+                      "weight must be (hidden,)");
+    w = weight->contiguous();
+    if (reinterpret_cast<uintptr_t>(w.data_ptr()) % 16) w = w.clone();
+    a.weight = w.data_ptr();
+    a.weight_dtype = float_dtype(w, "weight");
+    a.normed = normed.data_ptr();
+  } else {
+    a.weight_dtype = WMX_DTYPE_F32;
+  }
+  check_rc(wmx_residual_norm(&a, stream_of(x)), "wmx_residual_norm");
+  return normed;
+}
+
+// Queries (B, T, H * D) bf16 -> (B, T, H, D): rms_norm, weight, bf16, RoPE with
+// fp32 cos/sin (B, T, D), bf16.
+Tensor query_norm_rope(const Tensor& q, const Tensor& weight, const Tensor& cos, const Tensor& sin, int64_t heads, double eps) {
+  TORCH_CHECK_VALUE(q.dim() == 3 && q.scalar_type() == at::kBFloat16 && heads > 0 && q.size(2) % heads == 0,
+                    "query_norm_rope takes bfloat16 (B, T, H * D) queries");
+  const int64_t dim = q.size(2) / heads;
+  TORCH_CHECK_VALUE(cos.dim() == 3 && cos.size(0) == q.size(0) && cos.size(1) == q.size(1) && cos.size(2) == dim &&
+                        sin.sizes() == cos.sizes() && cos.scalar_type() == at::kFloat && sin.scalar_type() == at::kFloat &&
+                        weight.dim() == 1 && weight.size(0) == dim && cos.device() == q.device() &&
+                        sin.device() == q.device() && weight.device() == q.device(),
+                    "cos and sin must be float32 (B, T, D) and weight (D,) on the queries' device");
+  c10::OptionalDeviceGuard guard(q.device());
+  auto rows = [](const Tensor& t) {
+    const bool ok = t.stride(-1) == 1 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 && t.stride(0) % 4 == 0 &&
+                    t.stride(1) % 4 == 0;
+    return ok ? t : t.contiguous().clone();
+  };
+  Tensor c = rows(cos), s = rows(sin);
+  if (c.strides() != s.strides()) {
+    c = cos.contiguous().clone();
+    s = sin.contiguous().clone();
+  }
+  Tensor x = q.contiguous(), w = weight.contiguous();
+  if (reinterpret_cast<uintptr_t>(x.data_ptr()) % 16) x = x.clone();
+  if (reinterpret_cast<uintptr_t>(w.data_ptr()) % 16) w = w.clone();
+  Tensor out = at::empty({q.size(0), q.size(1), heads, dim}, q.options());
+  wmx_query_rope_args a;
+  std::memset(&a, 0, sizeof(a));
+  a.q = x.data_ptr();
+  a.weight = w.data_ptr();
+  a.weight_dtype = float_dtype(w, "weight");
+  a.cos = c.data_ptr<float>();
+  a.sin = s.data_ptr<float>();
+  a.out = out.data_ptr();
+  a.rope_stride[0] = c.stride(0);
+  a.rope_stride[1] = c.stride(1);
+  a.tokens = q.size(0) * q.size(1);
+  a.tokens_per_row = std::max<int64_t>(q.size(1), 1);
+  a.heads = (int32_t)heads;
+  a.head_dim = (int32_t)dim;
+  a.eps = (float)eps;
+  check_rc(wmx_query_norm_rope(&a, stream_of(q)), "wmx_query_norm_rope");
+  return out;
+}
+
+Tensor silu_mul(const Tensor& gate, const Tensor& up) {
+  TORCH_CHECK_VALUE(gate.sizes() == up.sizes() && gate.scalar_type() == at::kBFloat16 && up.scalar_type() == at::kBFloat16 &&
+                        gate.device() == up.device() && gate.numel() % 8 == 0,
+                    "silu_mul takes two bfloat16 tensors of one shape with a multiple of 8 elements");
+  c10::OptionalDeviceGuard guard(gate.device());
+  Tensor g = gate.contiguous(), u = up.contiguous();
+  if (reinterpret_cast<uintptr_t>(g.data_ptr()) % 16) g = g.clone();
+  if (reinterpret_cast<uintptr_t>(u.data_ptr()) % 16) u = u.clone();
+  Tensor out = at::empty(gate.sizes(), gate.options());
+  check_rc(wmx_silu_mul(g.data_ptr(), u.data_ptr(), out.data_ptr(), gate.numel(), stream_of(gate)), "wmx_silu_mul");
+  return out;
+}
+
 // ------------------------------------------------- strict autograd ----
 // Forward below the autograd key, saving what the backward operator reads;
 // gradients are returned in the inputs' dtypes.
@@ -1061,6 +1188,9 @@ TORCH_LIBRARY_FRAGMENT(white_matter, m) {
       "strict_decode_out(Tensor(a!) out, Tensor query, Tensor key, Tensor value, Tensor? query_start, "
       "int query_start_value, Tensor? kv_lengths, Tensor? key_mask, bool use_dummy, float scale, int num_splits) "
       "-> ()");
+  m.def("residual_norm(Tensor x, Tensor? delta, Tensor(a!)? out, Tensor? weight, float eps) -> Tensor");
+  m.def("query_norm_rope(Tensor q, Tensor weight, Tensor cos, Tensor sin, int heads, float eps) -> Tensor");
+  m.def("silu_mul(Tensor gate, Tensor up) -> Tensor");
   m.def("_packed_plan_cache_size() -> int", &packed_plan_cache_size);
   m.def("_packed_plan_cache_clear() -> ()", &packed_plan_cache_clear);
 }
@@ -1076,6 +1206,9 @@ TORCH_LIBRARY_IMPL(white_matter, CUDA, m) {
   m.impl("strict_dense_bwd", &strict_dense_bwd);
   m.impl("strict_decode", &strict_decode);
   m.impl("strict_decode_out", &strict_decode_out);
+  m.impl("residual_norm", &residual_norm);
+  m.impl("query_norm_rope", &query_norm_rope);
+  m.impl("silu_mul", &silu_mul);
 }
 
 TORCH_LIBRARY_IMPL(white_matter, Autograd, m) {

@@ -42,10 +42,28 @@ from dataclasses import dataclass
 import torch
 import torch.nn.functional as F
 
-from . import kv_pool
+from . import _native, kv_pool
 from .cyclic_attention import cyclic_attention
 from .metadata import prepare_feedback_metadata
 from .strict_causal_attention import strict_causal_attention
+
+
+# residual_norm, query_norm_rope and silu_mul (csrc/torch_ops.cpp, layer_ops.hip):
+# the token-local steps between a layer's products
+_native.load_ops()
+
+
+def _fake_residual_norm(x, delta, out, weight, eps):
+    return x.new_empty(x.shape if weight is not None else (0,), dtype=torch.bfloat16)
+
+
+def _fake_query_norm_rope(q, weight, cos, sin, heads, eps):
+    return q.new_empty(q.shape[0], q.shape[1], heads, q.shape[2] // heads)
+
+
+torch.library.register_fake("white_matter::residual_norm", _fake_residual_norm)
+torch.library.register_fake("white_matter::query_norm_rope", _fake_query_norm_rope)
+torch.library.register_fake("white_matter::silu_mul", lambda gate, up: torch.empty_like(gate))
 
 
 @dataclass(frozen=True)
@@ -198,10 +216,38 @@ class FeedbackModel:
         x = F.rms_norm(x.to(self.residual_dtype), (x.shape[-1],), None, eps)
         return (x * weight.to(self.residual_dtype)).to(self.dtype)
 
+    def _fused(self, x: torch.Tensor) -> bool:
+        """The layer's token-local steps run as HIP kernels: on the GPU without
+        gradients, bf16 activations over an fp32 residual stream, in the sizes
+        that the kernels take. Other models run the torch operations."""
+        c = self.config
+        return (
+            x.is_cuda and x.dtype == self.residual_dtype == torch.float32 and self.dtype == torch.bfloat16
+            and not torch.is_grad_enabled() and c.head_dim in (64, 96, 128) and c.hidden_size % 8 == 0
+            and c.hidden_size <= 4096 and c.intermediate_size % 8 == 0
+        )
+
+    def _layer_fused(self, index: int, h: torch.Tensor, x: torch.Tensor, out: torch.Tensor, attend, rope) -> torch.Tensor:
+        """The layer from its normed input h to the MLP's product, which the
+        caller adds to the residual stream: x the stream, `out` where x plus the
+        attention's output goes."""
+        c, p, ops = self.config, self.layers[index], torch.ops.white_matter
+        batch, length, _ = x.shape
+        q = ops.query_norm_rope(h @ p["q_proj"].t(), p["q_norm"], rope[0], rope[1], c.num_heads, c.rms_norm_eps)
+        a = attend(q.transpose(1, 2)).reshape(batch, length, c.num_heads * c.head_dim)
+        h = ops.residual_norm(x, a @ p["o_proj"].t(), out, p["post_norm"], c.rms_norm_eps)
+        return ops.silu_mul(h @ p["gate"].t(), h @ p["up"].t()) @ p["down"].t()
+
     def layer(self, index: int, x: torch.Tensor, attend, rope) -> torch.Tensor:
         """decoder_layer.py:51-72 with layers/white_matter.py:109-116, 199:
         x (B, T, d) residual; attend(q (B, Hq, T, D)) -> (B, T, Hq, D)."""
         c, p = self.config, self.layers[index]
+        if self._fused(x):
+            ops = torch.ops.white_matter
+            h = ops.residual_norm(x, None, None, p["input_norm"], c.rms_norm_eps)
+            mid, out = (torch.empty(x.shape, device=x.device, dtype=x.dtype) for _ in range(2))
+            ops.residual_norm(mid, self._layer_fused(index, h, x, mid, attend, rope), out, None, c.rms_norm_eps)
+            return out
         batch, length, _ = x.shape
         h = self._norm(x, p["input_norm"])
         q = (h @ p["q_proj"].t()).view(batch, length, c.num_heads, c.head_dim)
@@ -217,12 +263,34 @@ class FeedbackModel:
     def layers_forward(self, x: torch.Tensor, attend_layer, rope) -> tuple[torch.Tensor, list[torch.Tensor]]:
         """run_feedback_layers (decoder_layer.py:75-94) with the top output kept:
         returns the output and the L + 1 pool sources."""
+        if self._fused(x):
+            x, stacked = self.layers_stacked(x, attend_layer, rope)
+            return x, list(stacked.unbind(2))
         states = []
         for index in range(self.config.num_layers):
             states.append(x)
             x = self.layer(index, x, lambda q, i=index: attend_layer(i, q), rope)
         states.append(x)
         return x, states
+
+    def layers_stacked(self, x: torch.Tensor, attend_layer, rope) -> tuple[torch.Tensor, torch.Tensor]:
+        """`layers_forward` with the L + 1 pool sources as one (B, T, L + 1, d)
+        tensor. On the GPU the residual stream lives in it: each layer's last
+        add, with the next layer's norm, writes the next source."""
+        if not self._fused(x):
+            x, states = self.layers_forward(x, attend_layer, rope)
+            return x, torch.stack(states, dim=2)
+        c, ops, eps = self.config, torch.ops.white_matter, self.config.rms_norm_eps
+        batch, length, hidden = x.shape
+        stacked = torch.empty(batch, length, c.num_sources, hidden, device=x.device, dtype=x.dtype)
+        sources = stacked.unbind(2)
+        mid = torch.empty(x.shape, device=x.device, dtype=x.dtype)
+        h = ops.residual_norm(x, None, sources[0], self.layers[0]["input_norm"], eps)
+        for index in range(c.num_layers):
+            mlp = self._layer_fused(index, h, sources[index], mid, lambda q, i=index: attend_layer(i, q), rope)
+            last = index + 1 == c.num_layers
+            h = ops.residual_norm(mid, mlp, sources[index + 1], None if last else self.layers[index + 1]["input_norm"], eps)
+        return sources[-1], stacked
 
     def projection_inputs(self, stacked: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         """KVPool._project up to the projection (kv_pool.py:97-136, routing.py:
@@ -264,6 +332,9 @@ class FeedbackModel:
 
     def logits(self, x: torch.Tensor) -> torch.Tensor:
         """Tied output head on the final norm."""
+        if self._fused(x):
+            c = self.config
+            return torch.ops.white_matter.residual_norm(x, None, None, self.final_norm, c.rms_norm_eps) @ self.embed.t()
         return self._norm(x, self.final_norm) @ self.embed.t()
 
     def new_pool(self, batch: int, capacity: int) -> tuple[torch.Tensor, torch.Tensor]:
@@ -312,9 +383,9 @@ def cyclic_pass(model: FeedbackModel, x, keys, values, groups, rope, metadata=No
                 metadata=None if metadata is None else metadata[g],
             )
 
-        h, states = model.layers_forward(x.index_select(1, positions), attend, group_rope)
+        h, stacked = model.layers_stacked(x.index_select(1, positions), attend, group_rope)
         out.index_copy_(1, positions, h)
-        write_sources(model, torch.stack(states, dim=2), keys, values, positions + offset, group_rope, kernels)
+        write_sources(model, stacked, keys, values, positions + offset, group_rope, kernels)
     return out
 
 
@@ -443,9 +514,9 @@ class GreedyDecoder:
                 key_mask=self.key_mask,
             )
 
-        x, states = model.layers_forward(x, attend, rope)
+        x, stacked = model.layers_stacked(x, attend, rope)
         slot = self.length
-        key, value = model.project(torch.stack(states, dim=2), self.kernels)
+        key, value = model.project(stacked, self.kernels)
         self.kernels.store(key, value, model.k_norm, rope[0], rope[1], self.keys, self.values, slot,
                            eps=c.rms_norm_eps)
         self.key_mask.index_fill_(1, slot, True)
