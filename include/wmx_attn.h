@@ -39,7 +39,7 @@
 extern "C" {
 #endif
 
-#define WMX_ABI_VERSION 14
+#define WMX_ABI_VERSION 15
 
 enum {
   WMX_OK = 0,
@@ -572,6 +572,37 @@ typedef struct wmx_query_rope_args {
 } wmx_query_rope_args;
 
 /*
+ * The layer's products on a group's token rows, p = bf16(x weight^T) (bf16
+ * operands, fp32 sums), each with the token-local step that follows it:
+ *   WMX_LINEAR_PLAIN: out = p
+ *   WMX_LINEAR_GATED: wmx_silu_mul of p and bf16(x weight2^T)
+ *   WMX_LINEAR_QUERY: wmx_query_norm_rope of p, out_features = heads * head_dim
+ */
+#define WMX_LINEAR_PLAIN 0
+#define WMX_LINEAR_GATED 1
+#define WMX_LINEAR_QUERY 2
+typedef struct wmx_linear_args {
+  const void* x;              /* bf16 (rows, in_features), rows x_stride elements apart */
+  const void* weight;         /* bf16 (out_features, in_features) contiguous */
+  const void* weight2;        /* the same; WMX_LINEAR_GATED only */
+  void* out;                  /* bf16 (rows, out_features) contiguous */
+  int64_t x_stride;           /* in [in_features, 2^22), a multiple of 8 */
+  int64_t rows;
+  int32_t in_features;        /* multiples of 8, at least 8; in_features < 2^22 */
+  int32_t out_features;
+  int32_t kind;
+  /* WMX_LINEAR_QUERY only, as in wmx_query_rope_args */
+  int32_t head_dim;
+  int32_t norm_dtype;
+  float eps;
+  const void* norm;
+  const float* cos;
+  const float* sin;
+  int64_t rope_stride[2];
+  int64_t tokens_per_row;
+} wmx_linear_args;
+
+/*
  * Plans of packed attention calls on the device (the work lists, segment
  * fields and dS layout that wmx_attn_args takes). Two kinds of input:
  *   cyclic documents (q_seg != NULL): the int32 metadata of wmx_attn_args over
@@ -799,6 +830,7 @@ int wmx_kv_mix_bwd(const wmx_kv_mix_bwd_args* args, void* stream);
 int wmx_residual_norm(const wmx_residual_norm_args* args, void* stream);
 int wmx_query_norm_rope(const wmx_query_rope_args* args, void* stream);
 int wmx_silu_mul(const void* gate, const void* up, void* out, int64_t n, void* stream);
+int wmx_linear(const wmx_linear_args* args, void* stream);
 
 /* Plans of packed calls (see wmx_plan_args): no counterpart in the reference,
  * whose kernels take the metadata as it is. */

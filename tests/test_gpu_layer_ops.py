@@ -92,3 +92,47 @@ def test_layer_matches_the_torch_operations(tokens):
         eager.sum().backward()
     # a bf16 rounding moved in the norm reaches the layer's output through two products
     assert (fused - eager.detach()).norm() <= 2e-3 * (eager.detach() - x.detach()).norm()
+
+
+@pytest.mark.parametrize(
+    ("rows", "inner", "outer"),
+    [(1, 8, 8), (33, 136, 72), (64, 128, 64), (65, 1160, 200), (513, 264, 1032), (1100, 512, 1536)],
+)
+@torch.no_grad()
+def test_linear(rows, inner, outer):
+    """Plain and gated products, either side of both row tiles, with partial
+    stages and tiles, against float64. Bounds: one bf16 rounding of the result
+    and the fp32 sums' error, inner * 2^-24 of the sum of magnitudes."""
+    gen = torch.Generator(device=DEV).manual_seed(rows + inner)
+    wide = torch.randn(1, rows + 1, inner + 3, generator=gen, device=DEV).bfloat16()
+    x = wide[:, 1:, 3:]  # rows that the kernel cannot read in place
+    gate, up = (torch.randn(outer, inner, generator=gen, device=DEV).mul(inner**-0.5).bfloat16() for _ in range(2))
+    xd, gd, ud = x.double(), gate.double(), up.double()
+    p, u = xd @ gd.t(), xd @ ud.t()
+    slack = lambda w: inner * 2**-24 * (xd.abs() @ w.abs().t())  # noqa: E731
+    got = ops.linear_rows(x, gate)
+    assert got.shape == p.shape and ((got.double() - p).abs() <= 2**-8 * p.abs() + slack(gd)).all()
+    want = F.silu(p) * u
+    # both products, the activation (slope at most 1.1) and the result are rounded to bf16
+    bound = 1.1 * u.abs() * (2**-8 * p.abs() + slack(gd)) + F.silu(p).abs() * slack(ud) + 3 * 2**-8 * want.abs()
+    bound = 1.02 * bound + 1e-30  # (terms of second order, fp32 steps)
+    assert ((ops.linear_gated(x, gate, up).double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize(("batch", "length", "inner", "heads", "dim"), [(1, 1, 8, 1, 64), (3, 11, 200, 12, 96), (2, 33, 136, 3, 128), (5, 13, 512, 8, 64)])
+@torch.no_grad()
+def test_linear_query(batch, length, inner, heads, dim):
+    gen = torch.Generator(device=DEV).manual_seed(dim + inner)
+    x = torch.randn(batch, length, inner, generator=gen, device=DEV).bfloat16()
+    proj = torch.randn(heads * dim, inner, generator=gen, device=DEV).mul(inner**-0.5).bfloat16()
+    weight = (1 + 0.1 * torch.randn(dim, generator=gen, device=DEV)).bfloat16()
+    angle = torch.rand(batch, length + 2, dim // 2, generator=gen, device=DEV) * 50
+    cos, sin = (torch.cat((t, t), -1)[:, 1:-1] for t in (angle.cos(), angle.sin()))
+    got = ops.linear_query(x, proj, weight, cos, sin, heads, 1e-6)
+    q = (x.double() @ proj.double().t()).view(batch, length, heads, dim)
+    y = F.rms_norm(q, (dim,), None, 1e-6) * weight.double()
+    rot = torch.cat((-y[..., dim // 2 :], y[..., : dim // 2]), -1)
+    want = y * cos[:, :, None].double() + rot * sin[:, :, None].double()
+    # four bf16 roundings: the product, the mean through it, y and the result, 2^-8 of each term
+    assert got.shape == want.shape
+    assert ((got.double() - want).abs() <= (2**-6 + 2**-11) * (y.abs() + rot.abs()) + 1e-6).all()

@@ -19,7 +19,7 @@ import torch
 LIBRARY = Path(__file__).resolve().parent / "lib" / "libwmx_attn.so"
 # the operators registered from C++ (csrc/torch_ops.cpp), linked against LIBRARY
 OPS_LIBRARY = Path(__file__).resolve().parent / "lib" / "libwmx_torch.so"
-ABI_VERSION = 14
+ABI_VERSION = 15
 
 _c_i64_3 = ctypes.c_int64 * 3
 _c_i64_2 = ctypes.c_int64 * 2
@@ -423,6 +423,7 @@ EXPORTS = (
     "wmx_residual_norm",
     "wmx_query_norm_rope",
     "wmx_silu_mul",
+    "wmx_linear",
     "wmx_kv_mix_bwd_args_size",
     "wmx_kv_mix_bwd_workspace_size",
     "wmx_kv_mix_bwd",

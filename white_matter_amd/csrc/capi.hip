@@ -571,6 +571,34 @@ int wmx_silu_mul(const void* gate, const void* up, void* out, int64_t n, void* s
   return launched(wmx::launch_silu_mul(gate, up, out, n, (hipStream_t)stream));
 }
 
+int wmx_linear(const wmx_linear_args* a, void* stream) {
+  if (!a) return fail(WMX_E_INVALID, "args is NULL");
+  if (a->rows < 0 || a->in_features < 8 || a->in_features % 8 || a->in_features >= 1 << 22 || a->out_features < 8 ||
+      a->out_features % 8)
+    return fail(WMX_E_UNSUPPORTED, "linear features %d -> %d are not multiples of 8", a->in_features, a->out_features);
+  if (a->x_stride < a->in_features || a->x_stride % 8 || a->x_stride >= 1 << 22)
+    return fail(WMX_E_UNSUPPORTED, "linear rows must lie a multiple of 8, at least in_features, elements apart");
+  if (a->kind != WMX_LINEAR_PLAIN && a->kind != WMX_LINEAR_GATED && a->kind != WMX_LINEAR_QUERY)
+    return fail(WMX_E_INVALID, "linear kind %d", a->kind);
+  const bool query = a->kind == WMX_LINEAR_QUERY;
+  if (query) {
+    if (a->head_dim != 64 && a->head_dim != 96 && a->head_dim != 128)
+      return fail(WMX_E_UNSUPPORTED, "head_dim %d is not 64, 96 or 128", a->head_dim);
+    if (a->out_features % a->head_dim || a->tokens_per_row < 1) return fail(WMX_E_INVALID, "out_features must be heads of head_dim");
+    if (a->norm_dtype != WMX_DTYPE_F32 && a->norm_dtype != WMX_DTYPE_BF16)
+      return fail(WMX_E_INVALID, "dtype must be WMX_DTYPE_F32 or WMX_DTYPE_BF16");
+    if (!(a->eps >= 0.f)) return fail(WMX_E_INVALID, "eps must be >= 0");
+  }
+  if (a->rows == 0) return WMX_OK;
+  if (!a->x || !a->weight || !a->out || (a->kind == WMX_LINEAR_GATED && !a->weight2) ||
+      (query && (!a->norm || !a->cos || !a->sin)))
+    return fail(WMX_E_INVALID, "linear pointer is NULL");
+  if (!aligned16(a->x) || !aligned16(a->weight) || !aligned16(a->weight2) || !aligned16(a->out) ||
+      (query && (!aligned16(a->norm) || !aligned16(a->cos) || !aligned16(a->sin) || a->rope_stride[0] % 4 || a->rope_stride[1] % 4)))
+    return fail(WMX_E_INVALID, "linear operands must be 16-byte aligned rows");
+  return launched(wmx::launch_linear(*a, (hipStream_t)stream));
+}
+
 size_t wmx_plan_args_size(void) { return sizeof(wmx_plan_args); }
 
 int64_t wmx_plan_workspace_size(const wmx_plan_args* a) { return a ? wmx::plan_workspace_size(*a) : 0; }

@@ -246,13 +246,13 @@ struct TileDMA {
 // operations, and they complete in issue order), then the waves meet. The
 // empty asm statements keep the compiler from moving memory accesses across
 // the barrier; no global memory ordering is implied (the kernels exchange
-// data through LDS only). s_waitcnt immediate: vmcnt [3:0] (high bits
-// [15:14] zero), expcnt [6:4] = 7 (no wait), lgkmcnt [11:8] = 0.
+// data through LDS only). s_waitcnt immediate: vmcnt [3:0] and
+// [15:14], expcnt [6:4] = 7 (no wait), lgkmcnt [11:8] = 0.
 template <int VM = 0>
 __device__ __forceinline__ void lds_sync() {
-  static_assert(VM >= 0 && VM <= 15, "vmcnt immediate");
+  static_assert(VM >= 0 && VM <= 63, "vmcnt immediate");
   __asm__ volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(0x0070 | VM);
+  __builtin_amdgcn_s_waitcnt(0x0070 | (VM & 15) | (VM >> 4 << 14));
   __builtin_amdgcn_s_barrier();
   __asm__ volatile("" ::: "memory");
 }

@@ -989,28 +989,37 @@ Tensor residual_norm(const Tensor& x, const c10::optional<Tensor>& delta, const 
   return normed;
 }
 
+// The checked RoPE tables of tokens x (B, T, ...): c and s are cos and sin
+// with one pair of row strides and 16-byte aligned rows.
+void rope_rows(const Tensor& cos, const Tensor& sin, const Tensor& weight, const Tensor& x, int64_t dim, Tensor& c, Tensor& s) {
+  TORCH_CHECK_VALUE(cos.dim() == 3 && cos.size(0) == x.size(0) && cos.size(1) == x.size(1) && cos.size(2) == dim &&
+                        sin.sizes() == cos.sizes() && cos.scalar_type() == at::kFloat && sin.scalar_type() == at::kFloat &&
+                        weight.dim() == 1 && weight.size(0) == dim && cos.device() == x.device() &&
+                        sin.device() == x.device() && weight.device() == x.device(),
+                    "cos and sin must be float32 (B, T, D) and weight (D,) on the queries' device");
+  c10::OptionalDeviceGuard guard(x.device());
+  auto rows = [](const Tensor& t) {
+    const bool ok = t.stride(-1) == 1 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 && t.stride(0) % 4 == 0 &&
+                    t.stride(1) % 4 == 0;
+    return ok ? t : t.contiguous().clone();
+  };
+  c = rows(cos);
+  s = rows(sin);
+  if (c.strides() != s.strides()) {
+    c = cos.contiguous().clone();
+    s = sin.contiguous().clone();
+  }
+}
+
 // Queries (B, T, H * D) bf16 -> (B, T, H, D): rms_norm, weight, bf16, RoPE with
 // fp32 cos/sin (B, T, D), bf16.
 Tensor query_norm_rope(const Tensor& q, const Tensor& weight, const Tensor& cos, const Tensor& sin, int64_t heads, double eps) {
   TORCH_CHECK_VALUE(q.dim() == 3 && q.scalar_type() == at::kBFloat16 && heads > 0 && q.size(2) % heads == 0,
                     "query_norm_rope takes bfloat16 (B, T, H * D) queries");
   const int64_t dim = q.size(2) / heads;
-  TORCH_CHECK_VALUE(cos.dim() == 3 && cos.size(0) == q.size(0) && cos.size(1) == q.size(1) && cos.size(2) == dim &&
-                        sin.sizes() == cos.sizes() && cos.scalar_type() == at::kFloat && sin.scalar_type() == at::kFloat &&
-                        weight.dim() == 1 && weight.size(0) == dim && cos.device() == q.device() &&
-                        sin.device() == q.device() && weight.device() == q.device(),
-                    "cos and sin must be float32 (B, T, D) and weight (D,) on the queries' device");
+  Tensor c, s;
+  rope_rows(cos, sin, weight, q, dim, c, s);
   c10::OptionalDeviceGuard guard(q.device());
-  auto rows = [](const Tensor& t) {
-    const bool ok = t.stride(-1) == 1 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 && t.stride(0) % 4 == 0 &&
-                    t.stride(1) % 4 == 0;
-    return ok ? t : t.contiguous().clone();
-  };
-  Tensor c = rows(cos), s = rows(sin);
-  if (c.strides() != s.strides()) {
-    c = cos.contiguous().clone();
-    s = sin.contiguous().clone();
-  }
   Tensor x = q.contiguous(), w = weight.contiguous();
   if (reinterpret_cast<uintptr_t>(x.data_ptr()) % 16) x = x.clone();
   if (reinterpret_cast<uintptr_t>(w.data_ptr()) % 16) w = w.clone();
@@ -1044,6 +1053,90 @@ Tensor silu_mul(const Tensor& gate, const Tensor& up) {
   if (reinterpret_cast<uintptr_t>(u.data_ptr()) % 16) u = u.clone();
   Tensor out = at::empty(gate.sizes(), gate.options());
   check_rc(wmx_silu_mul(g.data_ptr(), u.data_ptr(), out.data_ptr(), gate.numel(), stream_of(gate)), "wmx_silu_mul");
+  return out;
+}
+
+// Contiguous and 16-byte aligned.
+Tensor dense16(const Tensor& t) {
+  Tensor c = t.contiguous();
+  return reinterpret_cast<uintptr_t>(c.data_ptr()) % 16 ? c.clone() : c;
+}
+
+// Products of bf16 rows x (..., in) with (out, in) weights (linear.hip): the
+// fields that every kind shares. x and weight must outlive the launch.
+void linear_args(wmx_linear_args& a, const Tensor& x, const Tensor& weight, const Tensor& out, int32_t kind) {
+  std::memset(&a, 0, sizeof(a));
+  a.x = x.data_ptr();
+  a.weight = weight.data_ptr();
+  a.out = out.data_ptr();
+  a.in_features = (int32_t)weight.size(1);
+  a.out_features = (int32_t)weight.size(0);
+  a.x_stride = a.in_features;
+  a.rows = x.numel() / weight.size(1);
+  a.kind = kind;
+}
+
+void check_linear(const Tensor& x, const Tensor& weight) {
+  TORCH_CHECK_VALUE(x.dim() >= 1 && x.scalar_type() == at::kBFloat16 && weight.dim() == 2 &&
+                        weight.scalar_type() == at::kBFloat16 && weight.size(1) == x.size(-1) && weight.device() == x.device() &&
+                        weight.size(0) > 0 && weight.size(1) > 0 && weight.size(0) <= INT32_MAX && weight.size(1) <= INT32_MAX,
+                    "a product takes bfloat16 rows (..., in) and a (out, in) weight on their device");
+}
+
+Tensor linear_out(const Tensor& x, int64_t features) {
+  auto sizes = x.sizes().vec();
+  sizes.back() = features;
+  return at::empty(sizes, x.options());
+}
+
+// x weight^T
+Tensor linear_rows(const Tensor& x, const Tensor& weight) {
+  check_linear(x, weight);
+  c10::OptionalDeviceGuard guard(x.device());
+  const Tensor rows = dense16(x), w = dense16(weight), out = linear_out(x, weight.size(0));
+  wmx_linear_args a;
+  linear_args(a, rows, w, out, WMX_LINEAR_PLAIN);
+  check_rc(wmx_linear(&a, stream_of(x)), "wmx_linear");
+  return out;
+}
+
+// silu(x gate^T) * (x up^T)
+Tensor linear_gated(const Tensor& x, const Tensor& gate, const Tensor& up) {
+  check_linear(x, gate);
+  check_linear(x, up);
+  TORCH_CHECK_VALUE(gate.sizes() == up.sizes(), "gate and up must have one shape");
+  c10::OptionalDeviceGuard guard(x.device());
+  const Tensor rows = dense16(x), g = dense16(gate), u = dense16(up), out = linear_out(x, gate.size(0));
+  wmx_linear_args a;
+  linear_args(a, rows, g, out, WMX_LINEAR_GATED);
+  a.weight2 = u.data_ptr();
+  check_rc(wmx_linear(&a, stream_of(x)), "wmx_linear");
+  return out;
+}
+
+// query_norm_rope of x weight^T: x (B, T, in), weight (H * D, in) -> (B, T, H, D).
+Tensor linear_query(const Tensor& x, const Tensor& weight, const Tensor& norm, const Tensor& cos, const Tensor& sin, int64_t heads,
+                    double eps) {
+  check_linear(x, weight);
+  TORCH_CHECK_VALUE(x.dim() == 3 && heads > 0 && weight.size(0) % heads == 0, "queries take rows (B, T, in) and a (H * D, in) weight");
+  const int64_t dim = weight.size(0) / heads;
+  Tensor c, s;
+  rope_rows(cos, sin, norm, x, dim, c, s);
+  c10::OptionalDeviceGuard guard(x.device());
+  const Tensor rows = dense16(x), w = dense16(weight), n = dense16(norm);
+  Tensor out = at::empty({x.size(0), x.size(1), heads, dim}, x.options());
+  wmx_linear_args a;
+  linear_args(a, rows, w, out, WMX_LINEAR_QUERY);
+  a.head_dim = (int32_t)dim;
+  a.norm = n.data_ptr();
+  a.norm_dtype = float_dtype(n, "weight");
+  a.eps = (float)eps;
+  a.cos = c.data_ptr<float>();
+  a.sin = s.data_ptr<float>();
+  a.rope_stride[0] = c.stride(0);
+  a.rope_stride[1] = c.stride(1);
+  a.tokens_per_row = std::max<int64_t>(x.size(1), 1);
+  check_rc(wmx_linear(&a, stream_of(x)), "wmx_linear");
   return out;
 }
 
@@ -1191,6 +1284,9 @@ TORCH_LIBRARY_FRAGMENT(white_matter, m) {
   m.def("residual_norm(Tensor x, Tensor? delta, Tensor(a!)? out, Tensor? weight, float eps) -> Tensor");
   m.def("query_norm_rope(Tensor q, Tensor weight, Tensor cos, Tensor sin, int heads, float eps) -> Tensor");
   m.def("silu_mul(Tensor gate, Tensor up) -> Tensor");
+  m.def("linear_rows(Tensor x, Tensor weight) -> Tensor");
+  m.def("linear_gated(Tensor x, Tensor gate, Tensor up) -> Tensor");
+  m.def("linear_query(Tensor x, Tensor weight, Tensor norm, Tensor cos, Tensor sin, int heads, float eps) -> Tensor");
   m.def("_packed_plan_cache_size() -> int", &packed_plan_cache_size);
   m.def("_packed_plan_cache_clear() -> ()", &packed_plan_cache_clear);
 }
@@ -1209,6 +1305,9 @@ TORCH_LIBRARY_IMPL(white_matter, CUDA, m) {
   m.impl("residual_norm", &residual_norm);
   m.impl("query_norm_rope", &query_norm_rope);
   m.impl("silu_mul", &silu_mul);
+  m.impl("linear_rows", &linear_rows);
+  m.impl("linear_gated", &linear_gated);
+  m.impl("linear_query", &linear_query);
 }
 
 TORCH_LIBRARY_IMPL(white_matter, Autograd, m) {

@@ -49,7 +49,8 @@ from .strict_causal_attention import strict_causal_attention
 
 
 # residual_norm, query_norm_rope and silu_mul (csrc/torch_ops.cpp, layer_ops.hip):
-# the token-local steps between a layer's products
+# the token-local steps between a layer's products; linear_rows, linear_gated and
+# linear_query (linear.hip): the products, with the step that follows them
 _native.load_ops()
 
 
@@ -64,6 +65,27 @@ def _fake_query_norm_rope(q, weight, cos, sin, heads, eps):
 torch.library.register_fake("white_matter::residual_norm", _fake_residual_norm)
 torch.library.register_fake("white_matter::query_norm_rope", _fake_query_norm_rope)
 torch.library.register_fake("white_matter::silu_mul", lambda gate, up: torch.empty_like(gate))
+torch.library.register_fake("white_matter::linear_rows", lambda x, weight: x.new_empty(*x.shape[:-1], weight.shape[0]))
+torch.library.register_fake("white_matter::linear_gated", lambda x, gate, up: x.new_empty(*x.shape[:-1], gate.shape[0]))
+torch.library.register_fake(
+    "white_matter::linear_query",
+    lambda x, weight, norm, cos, sin, heads, eps: x.new_empty(*x.shape[:-1], heads, weight.shape[0] // heads),
+)
+
+
+# Products of up to this many 64 x 64 output tiles run as the framework's own
+# kernels (linear.hip), larger ones, bound by the matrix cores, in the library: a
+# product or the queries with a tile per CU, the gated pair three times as many.
+# Us of GPU time, own and library, at the line and past it (the library's call
+# takes 19 us of host time besides, the pair's 44): 1024 x 1024 -> 1024 (256
+# tiles) 6.5 and 7.8, its queries 7.8 and 11.2, 2048 rows (512 tiles) 10.1 and
+# 9.8, 18 and 15; gated 1024 x 1024 -> 3072 (768 tiles) 25 and 32, 2048 rows 50 and 43.
+_PLAIN_TILES = 256
+_GATED_TILES = 768
+
+
+def _tiles(rows: int, features: int) -> int:
+    return (rows + 63) // 64 * ((features + 63) // 64)
 
 
 @dataclass(frozen=True)
@@ -233,10 +255,22 @@ class FeedbackModel:
         attention's output goes."""
         c, p, ops = self.config, self.layers[index], torch.ops.white_matter
         batch, length, _ = x.shape
-        q = ops.query_norm_rope(h @ p["q_proj"].t(), p["q_norm"], rope[0], rope[1], c.num_heads, c.rms_norm_eps)
+        rows = batch * length
+
+        def product(y, weight):
+            return ops.linear_rows(y, weight) if _tiles(rows, weight.shape[0]) <= _PLAIN_TILES else y @ weight.t()
+
+        if _tiles(rows, p["q_proj"].shape[0]) <= _PLAIN_TILES:
+            q = ops.linear_query(h, p["q_proj"], p["q_norm"], rope[0], rope[1], c.num_heads, c.rms_norm_eps)
+        else:
+            q = ops.query_norm_rope(h @ p["q_proj"].t(), p["q_norm"], rope[0], rope[1], c.num_heads, c.rms_norm_eps)
         a = attend(q.transpose(1, 2)).reshape(batch, length, c.num_heads * c.head_dim)
-        h = ops.residual_norm(x, a @ p["o_proj"].t(), out, p["post_norm"], c.rms_norm_eps)
-        return ops.silu_mul(h @ p["gate"].t(), h @ p["up"].t()) @ p["down"].t()
+        h = ops.residual_norm(x, product(a, p["o_proj"]), out, p["post_norm"], c.rms_norm_eps)
+        if _tiles(rows, p["gate"].shape[0]) <= _GATED_TILES:
+            h = ops.linear_gated(h, p["gate"], p["up"])
+        else:
+            h = ops.silu_mul(h @ p["gate"].t(), h @ p["up"].t())
+        return product(h, p["down"])
 
     def layer(self, index: int, x: torch.Tensor, attend, rope) -> torch.Tensor:
         """decoder_layer.py:51-72 with layers/white_matter.py:109-116, 199:
