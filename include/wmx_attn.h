@@ -603,6 +603,23 @@ typedef struct wmx_linear_args {
 } wmx_linear_args;
 
 /*
+ * The pool's channel projections of both sides (reference modules/kv_pool.py:
+ * 137-160): out[c] = bf16(x[c] weight[c]), fp32 sums. All bf16 and contiguous.
+ */
+typedef struct wmx_pool_project_args {
+  const void* x_k;            /* (channels, rows, in_features) */
+  const void* x_v;
+  const void* weight_k;       /* (channels, in_features, out_features) */
+  const void* weight_v;
+  void* out_k;                /* (channels, rows, out_features) */
+  void* out_v;
+  int64_t rows;
+  int32_t channels;           /* at most 32767 */
+  int32_t in_features;        /* multiples of 8, in [8, 2^22) */
+  int32_t out_features;
+} wmx_pool_project_args;
+
+/*
  * Plans of packed attention calls on the device (the work lists, segment
  * fields and dS layout that wmx_attn_args takes). Two kinds of input:
  *   cyclic documents (q_seg != NULL): the int32 metadata of wmx_attn_args over
@@ -831,6 +848,7 @@ int wmx_residual_norm(const wmx_residual_norm_args* args, void* stream);
 int wmx_query_norm_rope(const wmx_query_rope_args* args, void* stream);
 int wmx_silu_mul(const void* gate, const void* up, void* out, int64_t n, void* stream);
 int wmx_linear(const wmx_linear_args* args, void* stream);
+int wmx_pool_project(const wmx_pool_project_args* args, void* stream);
 
 /* Plans of packed calls (see wmx_plan_args): no counterpart in the reference,
  * whose kernels take the metadata as it is. */

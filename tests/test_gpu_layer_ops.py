@@ -136,3 +136,16 @@ def test_linear_query(batch, length, inner, heads, dim):
     # four bf16 roundings: the product, the mean through it, y and the result, 2^-8 of each term
     assert got.shape == want.shape
     assert ((got.double() - want).abs() <= (2**-6 + 2**-11) * (y.abs() + rot.abs()) + 1e-6).all()
+
+
+@pytest.mark.parametrize(("channels", "rows", "inner", "outer"), [(1, 1, 8, 8), (3, 65, 136, 264), (2, 64, 128, 128), (8, 130, 1160, 512)])
+@torch.no_grad()
+def test_pool_project(channels, rows, inner, outer):
+    gen = torch.Generator(device=DEV).manual_seed(rows + inner)
+    x = [torch.randn(channels, rows, inner, generator=gen, device=DEV).bfloat16() for _ in range(2)]
+    w = [torch.randn(channels, inner, outer, generator=gen, device=DEV).mul(inner**-0.5).bfloat16() for _ in range(2)]
+    for got, a, b in zip(ops.pool_project(*x, *w), x, w, strict=True):
+        a, b = a.double(), b.double()
+        want = torch.bmm(a, b)
+        # one bf16 rounding and the fp32 sums
+        assert got.shape == want.shape and ((got.double() - want).abs() <= 2**-8 * want.abs() + inner * 2**-24 * torch.bmm(a.abs(), b.abs())).all()

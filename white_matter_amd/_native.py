@@ -424,6 +424,7 @@ EXPORTS = (
     "wmx_query_norm_rope",
     "wmx_silu_mul",
     "wmx_linear",
+    "wmx_pool_project",
     "wmx_kv_mix_bwd_args_size",
     "wmx_kv_mix_bwd_workspace_size",
     "wmx_kv_mix_bwd",

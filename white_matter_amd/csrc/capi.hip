@@ -599,6 +599,18 @@ int wmx_linear(const wmx_linear_args* a, void* stream) {
   return launched(wmx::launch_linear(*a, (hipStream_t)stream));
 }
 
+int wmx_pool_project(const wmx_pool_project_args* a, void* stream) {
+  if (!a) return fail(WMX_E_INVALID, "args is NULL");
+  if (a->rows < 0 || a->channels < 1 || a->channels > 32767) return fail(WMX_E_INVALID, "pool projection shape");
+  for (const int n : {a->in_features, a->out_features})
+    if (n < 8 || n % 8 || n >= 1 << 22)
+      return fail(WMX_E_UNSUPPORTED, "projection features %d -> %d are not multiples of 8", a->in_features, a->out_features);
+  if (a->rows == 0) return WMX_OK;
+  for (const void* p : {a->x_k, a->x_v, a->weight_k, a->weight_v, (const void*)a->out_k, (const void*)a->out_v})
+    if (!p || !aligned16(p)) return fail(WMX_E_INVALID, "projection operands must be 16-byte aligned");
+  return launched(wmx::launch_pool_project(*a, (hipStream_t)stream));
+}
+
 size_t wmx_plan_args_size(void) { return sizeof(wmx_plan_args); }
 
 int64_t wmx_plan_workspace_size(const wmx_plan_args* a) { return a ? wmx::plan_workspace_size(*a) : 0; }

@@ -341,6 +341,103 @@ __global__ __launch_bounds__(256, WT <= 2 ? 2 : 1) void linear_small_kernel(cons
 #endif
 }
 
+// The pool's channel projections, out[c] = x[c] W[c] with W (in, out) rows, both
+// sides of every channel in one launch: 64 rows by 128 columns. A stage's weight
+// rows are the contraction, read transposed from LDS (ds_read_b64_tr_b16); the
+// rows' operand is read in the same order of k. The two batched library products
+// take 36 us of host time, this launch 6. GPU time, before and here, in us, of
+// both sides: four channels of 512 -> 256, 16 rows 17.4 and 5.9, 1,024 rows 14.6
+// and 7.0; eight of 1024 -> 512, 16 rows 10.0 and 8.9, 512 rows 23.0 and 21.4.
+__global__ __launch_bounds__(256, 1) void pool_project_kernel(const wmx_pool_project_args a) {
+#ifdef __HIP_DEVICE_COMPILE__
+  constexpr int BM = kTileRows, BN = kRowElems, NS = 3, kStage = 3 * kTileElems;
+  __shared__ __attribute__((aligned(1024))) bf16 s0[kStage];
+  __shared__ __attribute__((aligned(1024))) bf16 s1[kStage];
+  __shared__ __attribute__((aligned(1024))) bf16 s2[kStage];
+  int64_t m0;
+  int n0;
+  if (!decode_tile(a.rows, a.out_features, BM, BN, m0, n0)) return;
+  const int side = blockIdx.y & 1;
+  const int64_t ch = blockIdx.y >> 1;
+  const int K = a.in_features, N = a.out_features;
+  const bf16* const weight = (const bf16*)(side ? a.weight_v : a.weight_k) + ch * K * N + n0;
+  bf16* const orow = (bf16*)(side ? a.out_v : a.out_k) + (ch * a.rows + m0) * N + n0;
+  const int mrows = (int)min((int64_t)BM, a.rows - m0), cols = min(BN, N - n0);
+  const int lane = threadIdx.x & 63, wave = wave_id(), half = lane >> 5, col = lane & 31;
+  const int wm = wave & 1, wn = wave >> 1;
+
+  using Tile = Operand<BM>;
+  typename Tile::DMA dma;
+  dma.init(wave, lane);
+  Tile x;
+  x.init(dma, (const bf16*)(side ? a.x_v : a.x_k) + ch * a.rows * K, m0, K, a.rows, K);
+  unsigned woff[Tile::DMA::kInstr];
+  dma.strided_offsets(N * 2, woff);
+#pragma unroll
+  for (int r = 0; r < Tile::DMA::kInstr; ++r) woff[r] = dma.chunk16(r) < 2 * cols ? woff[r] : kOutOfRange;
+  auto issue = [&](int kt, bf16* st) __attribute__((always_inline)) {
+    x.issue(dma, kt, st);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int k0 = kt * kStep + 64 * j, left = min(64, K - k0);
+      dma.issue_strided(make_rsrc(weight + (left > 0 ? (int64_t)k0 * N : 0), left > 0 ? ((left - 1) * N + cols) * 2 : 0),
+                        st + (1 + j) * kTileElems, woff);
+    }
+  };
+  TrReads<2> wr;
+  wr.init(lane, 64 * wn);
+  const int swz = tile_swz(col);
+  f32x16 acc[2] = {f32x16{}, f32x16{}};
+  issue(0, s0);
+  issue(1, s1);
+  for_stages<NS>((K + kStep - 1) / kStep, [&](auto bufc, int it) __attribute__((always_inline)) {
+    constexpr int B = decltype(bufc)::value, BX = (B + NS - 1) % NS;
+    lds_sync<(NS - 2) * 3 * Tile::DMA::kInstr>();
+    issue(it + NS - 1, BX == 0 ? s0 : BX == 1 ? s1 : s2);
+    const bf16* const st = B == 0 ? s0 : B == 1 ? s1 : s2;
+    const bf16* const xr = st + (32 * wm + col) * kRowElems + 4 * half;
+    wr.refresh();
+    constexpr int KS = kStep / 16, PF = 3;
+    bf16x8 xo[KS], wo[KS][2];
+    auto fetch = [&](int s) __attribute__((always_inline)) {
+      // k of element e: 16 s + 8 (e / 4) + 4 half + e % 4, as the transposed reads'
+      const u32x2 lo = *reinterpret_cast<const u32x2*>(xr + 8 * ((2 * s) ^ swz));
+      const u32x2 hi = *reinterpret_cast<const u32x2*>(xr + 8 * ((2 * s + 1) ^ swz));
+      xo[s] = as_bf16x8(u32x4{lo[0], lo[1], hi[0], hi[1]});
+#pragma unroll
+      for (int d = 0; d < 2; ++d) wo[s][d] = wr.get(st + (1 + s / 4) * kTileElems, d, s % 4);
+    };
+#pragma unroll
+    for (int s = 0; s < PF; ++s) fetch(s);
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (s + PF < KS) fetch(s + PF);
+#pragma unroll
+      for (int d = 0; d < 2; ++d) acc[d] = mfma32(wo[s][d], xo[s], acc[d]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  });
+  dma_barrier();  // every wave is done with the stages: the tile's rows are laid out in the first
+
+  // acc[d][r] is row 32 wm + col, column 64 wn + 32 d + 8 (r / 4) + 4 half + r % 4
+  constexpr int P = BN + 8;  // pitch
+  bf16* const mine = s0 + (32 * wm + col) * P + 64 * wn + 4 * half;
+#pragma unroll
+  for (int d = 0; d < 2; ++d)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<u32x2*>(mine + 32 * d + 8 * g) =
+          u32x2{pack_bf16x2(acc[d][4 * g], acc[d][4 * g + 1]), pack_bf16x2(acc[d][4 * g + 2], acc[d][4 * g + 3])};
+  lds_barrier();
+#pragma unroll
+  for (int i = threadIdx.x; i < BM * 16; i += 256) {
+    const int r = i >> 4, c = 8 * (i & 15);
+    if (r < mrows && c < cols) *reinterpret_cast<u32x4*>(orow + (int64_t)r * N + c) = *reinterpret_cast<const u32x4*>(s0 + r * P + c);
+  }
+#endif
+}
+
 int64_t grid_of(int64_t rows, int64_t cols) { return (rows * cols + kXcds - 1) / kXcds * kXcds; }
 
 template <int WT, int NS>
@@ -383,6 +480,13 @@ int launch_linear(const wmx_linear_args& a, hipStream_t stream) {
   const bool few = (a.rows + 63) / 64 * ((a.out_features + 63) / 64) <= kFewTiles;
   if (a.kind == WMX_LINEAR_GATED) return few ? run_small<WMX_LINEAR_GATED, 2, 3>(a, stream) : run<2, 3>(a, stream);
   return few ? run_small<WMX_LINEAR_PLAIN, 1, 4>(a, stream) : run<1, 4>(a, stream);
+}
+
+int launch_pool_project(const wmx_pool_project_args& a, hipStream_t stream) {
+  const int64_t grid = grid_of((a.rows + 63) / 64, (a.out_features + kRowElems - 1) / kRowElems);
+  if (grid > INT32_MAX) return WMX_E_UNSUPPORTED;
+  hipLaunchKernelGGL(pool_project_kernel, dim3((unsigned)grid, 2 * a.channels), dim3(256), 0, stream, a);
+  return WMX_OK;
 }
 
 }  // namespace wmx

@@ -1114,6 +1114,33 @@ Tensor linear_gated(const Tensor& x, const Tensor& gate, const Tensor& up) {
   return out;
 }
 
+// (channels, rows, in) rows times (channels, in, out) weights, both sides.
+std::tuple<Tensor, Tensor> pool_project(const Tensor& x_k, const Tensor& x_v, const Tensor& w_k, const Tensor& w_v) {
+  TORCH_CHECK_VALUE(x_k.dim() == 3 && w_k.dim() == 3 && x_v.sizes() == x_k.sizes() && w_v.sizes() == w_k.sizes() &&
+                        w_k.size(0) == x_k.size(0) && w_k.size(1) == x_k.size(2) && w_k.size(1) <= INT32_MAX &&
+                        w_k.size(2) <= INT32_MAX && x_k.size(0) <= INT32_MAX,
+                    "the projections take (k, rows, in) rows and (k, in, out) weights for each side");
+  for (const Tensor* t : {&x_k, &x_v, &w_k, &w_v})
+    TORCH_CHECK_VALUE(t->scalar_type() == at::kBFloat16 && t->device() == x_k.device(), "the projections take bfloat16 on one device");
+  c10::OptionalDeviceGuard guard(x_k.device());
+  const Tensor xk = dense16(x_k), xv = dense16(x_v), wk = dense16(w_k), wv = dense16(w_v);
+  Tensor out_k = at::empty({x_k.size(0), x_k.size(1), w_k.size(2)}, x_k.options()), out_v = at::empty_like(out_k);
+  wmx_pool_project_args a;
+  std::memset(&a, 0, sizeof(a));
+  a.x_k = xk.data_ptr();
+  a.x_v = xv.data_ptr();
+  a.weight_k = wk.data_ptr();
+  a.weight_v = wv.data_ptr();
+  a.out_k = out_k.data_ptr();
+  a.out_v = out_v.data_ptr();
+  a.rows = x_k.size(1);
+  a.channels = (int32_t)x_k.size(0);
+  a.in_features = (int32_t)w_k.size(1);
+  a.out_features = (int32_t)w_k.size(2);
+  check_rc(wmx_pool_project(&a, stream_of(x_k)), "wmx_pool_project");
+  return {out_k, out_v};
+}
+
 // query_norm_rope of x weight^T: x (B, T, in), weight (H * D, in) -> (B, T, H, D).
 Tensor linear_query(const Tensor& x, const Tensor& weight, const Tensor& norm, const Tensor& cos, const Tensor& sin, int64_t heads,
                     double eps) {
@@ -1286,6 +1313,7 @@ TORCH_LIBRARY_FRAGMENT(white_matter, m) {
   m.def("silu_mul(Tensor gate, Tensor up) -> Tensor");
   m.def("linear_rows(Tensor x, Tensor weight) -> Tensor");
   m.def("linear_gated(Tensor x, Tensor gate, Tensor up) -> Tensor");
+  m.def("pool_project(Tensor x_k, Tensor x_v, Tensor w_k, Tensor w_v) -> (Tensor, Tensor)");
   m.def("linear_query(Tensor x, Tensor weight, Tensor norm, Tensor cos, Tensor sin, int heads, float eps) -> Tensor");
   m.def("_packed_plan_cache_size() -> int", &packed_plan_cache_size);
   m.def("_packed_plan_cache_clear() -> ()", &packed_plan_cache_clear);
@@ -1308,6 +1336,7 @@ TORCH_LIBRARY_IMPL(white_matter, CUDA, m) {
   m.impl("linear_rows", &linear_rows);
   m.impl("linear_gated", &linear_gated);
   m.impl("linear_query", &linear_query);
+  m.impl("pool_project", &pool_project);
 }
 
 TORCH_LIBRARY_IMPL(white_matter, Autograd, m) {

@@ -74,6 +74,7 @@ int64_t feedback_meta_workspace_size(const wmx_feedback_meta_args& a);
 int launch_feedback_meta(const wmx_feedback_meta_args& a, hipStream_t stream);
 int64_t kv_mix_bwd_workspace_size(const wmx_kv_mix_bwd_args& a);
 int launch_kv_mix_bwd(const wmx_kv_mix_bwd_args& a, hipStream_t stream);
+int launch_pool_project(const wmx_pool_project_args& a, hipStream_t stream);
 int launch_linear(const wmx_linear_args& a, hipStream_t stream);
 int launch_residual_norm(const wmx_residual_norm_args& a, hipStream_t stream);
 int launch_query_norm_rope(const wmx_query_rope_args& a, hipStream_t stream);

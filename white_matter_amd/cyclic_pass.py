@@ -68,6 +68,10 @@ torch.library.register_fake("white_matter::silu_mul", lambda gate, up: torch.emp
 torch.library.register_fake("white_matter::linear_rows", lambda x, weight: x.new_empty(*x.shape[:-1], weight.shape[0]))
 torch.library.register_fake("white_matter::linear_gated", lambda x, gate, up: x.new_empty(*x.shape[:-1], gate.shape[0]))
 torch.library.register_fake(
+    "white_matter::pool_project",
+    lambda x_k, x_v, w_k, w_v: tuple(x_k.new_empty(*x_k.shape[:2], w_k.shape[2]) for _ in range(2)),
+)
+torch.library.register_fake(
     "white_matter::linear_query",
     lambda x, weight, norm, cos, sin, heads, eps: x.new_empty(*x.shape[:-1], heads, weight.shape[0] // heads),
 )
@@ -82,6 +86,9 @@ torch.library.register_fake(
 # 9.8, 18 and 15; gated 1024 x 1024 -> 3072 (768 tiles) 25 and 32, 2048 rows 50 and 43.
 _PLAIN_TILES = 256
 _GATED_TILES = 768
+# The pool's channel projections, of both sides together: 8 x 512 x 1024 -> 512
+# (1,024 tiles, two workgroups a CU) 21 and 23, 1,024 rows 39 and 30.
+_POOL_TILES = 1024
 
 
 def _tiles(rows: int, features: int) -> int:
@@ -356,13 +363,15 @@ class FeedbackModel:
         batch, length = stacked.shape[:2]
         mix = getattr(kernels, "mix", None)
         rows = mix(self, stacked) if mix is not None else self.projection_inputs(stacked)
-        out = []
-        for side, r in zip("kv", rows, strict=True):
-            proj = torch.bmm(r, self.proj[side])  # (k, B T, Hkv D)
-            out.append(
-                proj.view(c.num_kv_channels, batch, length, c.num_kv_heads, c.head_dim).permute(1, 0, 3, 2, 4)
-            )
-        return out[0], out[1]
+        width = c.num_kv_heads * c.head_dim
+        few = 2 * c.num_kv_channels * _tiles(batch * length, width) <= _POOL_TILES
+        if few and self._fused(stacked) and rows[0].dtype == torch.bfloat16:
+            projected = torch.ops.white_matter.pool_project(*rows, self.proj["k"], self.proj["v"])
+        else:
+            projected = [torch.bmm(r, self.proj[side]) for side, r in zip("kv", rows, strict=True)]  # (k, B T, Hkv D)
+        shape = (c.num_kv_channels, batch, length, c.num_kv_heads, c.head_dim)
+        key, value = (p.view(shape).permute(1, 0, 3, 2, 4) for p in projected)
+        return key, value
 
     def logits(self, x: torch.Tensor) -> torch.Tensor:
         """Tied output head on the final norm."""
