@@ -1,5 +1,5 @@
-"""The layer's fused steps (white_matter::residual_norm, query_norm_rope,
-silu_mul; csrc/layer_ops.hip) against the torch operations they replace, at the
+"""The layer's fused steps and products (white_matter::residual_norm, query_norm_rope,
+silu_mul, linear_*, pool_project) against the torch operations they replace, at the
 edges of their row and lane splits, and a model layer through them against the
 same layer through the torch operations.
 
@@ -11,6 +11,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
+from white_matter_amd import cyclic_pass
 from white_matter_amd.cyclic_pass import FeedbackConfig, FeedbackModel
 
 pytestmark = pytest.mark.gpu
@@ -149,3 +150,31 @@ def test_pool_project(channels, rows, inner, outer):
         want = torch.bmm(a, b)
         # one bf16 rounding and the fp32 sums
         assert got.shape == want.shape and ((got.double() - want).abs() <= 2**-8 * want.abs() + inner * 2**-24 * torch.bmm(a.abs(), b.abs())).all()
+
+
+@pytest.mark.parametrize(("tokens", "dim", "strided"), [(1, 96, False), (37, 128, True), (70, 64, True)])
+@torch.no_grad()
+def test_own_products_match_the_library(monkeypatch, tokens, dim, strided):
+    """A layer and the pool projection on either side of the size rule, with
+    weights that lie otherwise than the kernels read them."""
+    config = FeedbackConfig(vocab_size=64, hidden_size=136, intermediate_size=264, num_layers=2, num_heads=4, num_kv_heads=2,
+                            head_dim=dim, num_kv_channels=2)
+    model = FeedbackModel(config, device=DEV, seed=3)
+    if strided:
+        p = model.layers[0]
+        for name in ("q_proj", "o_proj", "gate", "up", "down"):
+            p[name] = p[name].t().contiguous().t()
+        model.proj = {side: torch.cat((w, w), -1)[..., : w.shape[-1]] for side, w in model.proj.items()}
+    gen = torch.Generator(device=DEV).manual_seed(4)
+    x = torch.randn(2, tokens, 136, generator=gen, device=DEV)
+    stacked = torch.randn(2, tokens, 3, 136, generator=gen, device=DEV)
+    rope = model.rope(torch.arange(tokens, device=DEV).expand(2, tokens))
+    run = lambda: (model.layer(0, x, lambda q: q.transpose(1, 2) * 0.5, rope), *model.project(stacked))  # noqa: E731
+    own = run()
+    for name in ("_PLAIN_TILES", "_GATED_TILES", "_POOL_TILES"):
+        monkeypatch.setattr(cyclic_pass, name, 0)
+    library = run()
+    # sums in another order move bf16 roundings, which reach the layer's output through two products
+    assert (own[0] - library[0]).norm() <= 2e-3 * (library[0] - x).norm()
+    for a, b in zip(own[1:], library[1:], strict=True):
+        _near(a, b, "projection")
