@@ -9,6 +9,7 @@ rounding boundary: one bf16 step (2^-7 relative at most), on few elements."""
 
 import pytest
 import torch
+import torch.autograd.forward_ad as fwAD
 import torch.nn.functional as F
 
 from white_matter_amd import cyclic_pass
@@ -178,3 +179,62 @@ def test_own_products_match_the_library(monkeypatch, tokens, dim, strided):
     assert (own[0] - library[0]).norm() <= 2e-3 * (library[0] - x).norm()
     for a, b in zip(own[1:], library[1:], strict=True):
         _near(a, b, "projection")
+
+
+def _small_model(tokens, seed=5, **config):
+    config = FeedbackConfig(vocab_size=64, hidden_size=136, intermediate_size=264, num_layers=2, num_heads=4, num_kv_heads=2,
+                            head_dim=64, num_kv_channels=2, **config)
+    gen = torch.Generator(device=DEV).manual_seed(seed)
+    x, t = (torch.randn(2, tokens, 136, generator=gen, device=DEV) for _ in range(2))
+    return FeedbackModel(config, device=DEV, seed=seed), x, t
+
+
+def _attend(q):
+    return q.transpose(1, 2) * 0.5
+
+
+@pytest.mark.parametrize("call", ["layer", "layers_forward", "layers_stacked", "logits"])
+def test_forward_mode_and_vmap_without_gradients(call):
+    """Tangents and batched inputs pass through the model as with gradients on,
+    where the torch operations run. The results are equal; a tangent and a
+    vmapped call are within 2^-8, one bf16 rounding of every element: torch's
+    derivative formulas and products differ in fp32 with gradients on, under
+    jvp, for dual numbers and in a batch, which moves their bf16 roundings."""
+    model, x, t = _small_model(5)
+    rope = model.rope(torch.arange(5, device=DEV).expand(2, 5))
+    fn = {
+        "layer": lambda x: model.layer(0, x, _attend, rope),
+        "layers_forward": lambda x: model.layers_forward(x, lambda i, q: _attend(q), rope)[0],
+        "layers_stacked": lambda x: model.layers_stacked(x, lambda i, q: _attend(q), rope)[1],
+        "logits": model.logits,
+    }[call]
+    near = lambda a, b: (a.float() - b.float()).norm() <= 2**-8 * b.float().norm()  # noqa: E731
+    want, tangent = torch.func.jvp(fn, (x,), (t,))
+    assert tangent.abs().max() > 0
+    with torch.no_grad():
+        got = torch.func.jvp(fn, (x,), (t,))
+        assert torch.equal(got[0], want) and near(got[1], tangent)
+        with fwAD.dual_level():
+            dual = fwAD.unpack_dual(fn(fwAD.make_dual(x, t)))
+            assert dual.tangent is not None, "the tangent was dropped"
+            assert torch.equal(dual.primal, want) and near(dual.tangent, tangent)
+        batched = torch.func.vmap(fn)(torch.stack((x, t)))
+    for one, row in zip(batched, (x, t), strict=True):
+        assert near(one, fn(row))
+
+
+@torch.no_grad()
+def test_tangents_of_weights_and_tables_without_gradients():
+    """A tangent that only a weight, the RoPE tables or the attention carries."""
+    model, x, _ = _small_model(5)
+    cos, sin = model.rope(torch.arange(5, device=DEV).expand(2, 5))
+    p = model.layers[0]
+    with fwAD.dual_level():
+        tangent = lambda attend, rope: fwAD.unpack_dual(model.layer(0, x, attend, rope)).tangent  # noqa: E731
+        assert tangent(_attend, (cos, sin)) is None
+        assert tangent(_attend, (fwAD.make_dual(cos, torch.ones_like(cos)), sin)) is not None
+        assert tangent(lambda q: fwAD.make_dual(_attend(q).contiguous(), torch.ones(2, 5, 4, 64, device=DEV).bfloat16()), (cos, sin)) is not None
+        kept = p["up"]
+        p["up"] = fwAD.make_dual(kept, torch.ones_like(kept))
+        assert tangent(_attend, (cos, sin)) is not None
+        p["up"] = kept

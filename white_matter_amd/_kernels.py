@@ -12,6 +12,7 @@ from __future__ import annotations
 from dataclasses import dataclass
 
 import torch
+import torch.autograd.forward_ad as forward_ad
 
 from . import _native
 
@@ -28,6 +29,16 @@ def guard_capture(what: str) -> None:
             f"{what} synchronises with the host, which HIP graph capture forbids; "
             "run the same call once before capturing so its schedule is cached"
         )
+
+
+def transformed() -> bool:
+    """Whether the caller runs under a functorch transform (vmap, jvp, the
+    batched backward of is_grads_batched) or inside a forward-mode dual level.
+    Disabling gradients disables neither, and any tensor of the call (an input,
+    a weight, what a callback returns) may be batched or carry a tangent there:
+    operators without a rule for them would refuse it or drop the tangent, so
+    the torch operations run."""
+    return torch._C._are_functorch_transforms_active() or forward_ad._current_level >= 0
 
 
 def kernel_head_dim(dim: int) -> int | None:

@@ -42,7 +42,7 @@ from dataclasses import dataclass
 import torch
 import torch.nn.functional as F
 
-from . import _native, kv_pool
+from . import _kernels, _native, kv_pool
 from .cyclic_attention import cyclic_attention
 from .metadata import prepare_feedback_metadata
 from .strict_causal_attention import strict_causal_attention
@@ -247,13 +247,14 @@ class FeedbackModel:
 
     def _fused(self, x: torch.Tensor) -> bool:
         """The layer's token-local steps run as HIP kernels: on the GPU without
-        gradients, bf16 activations over an fp32 residual stream, in the sizes
-        that the kernels take. Other models run the torch operations."""
+        gradients (forward-mode ones included) and vmap, bf16 activations over an
+        fp32 residual stream, in the sizes that the kernels take. Other calls run
+        the torch operations."""
         c = self.config
         return (
             x.is_cuda and x.dtype == self.residual_dtype == torch.float32 and self.dtype == torch.bfloat16
-            and not torch.is_grad_enabled() and c.head_dim in (64, 96, 128) and c.hidden_size % 8 == 0
-            and c.hidden_size <= 4096 and c.intermediate_size % 8 == 0
+            and not torch.is_grad_enabled() and not _kernels.transformed() and c.head_dim in (64, 96, 128)
+            and c.hidden_size % 8 == 0 and c.hidden_size <= 4096 and c.intermediate_size % 8 == 0
         )
 
     def _layer_fused(self, index: int, h: torch.Tensor, x: torch.Tensor, out: torch.Tensor, attend, rope) -> torch.Tensor:
