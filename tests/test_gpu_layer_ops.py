@@ -238,3 +238,30 @@ def test_tangents_of_weights_and_tables_without_gradients():
         p["up"] = fwAD.make_dual(kept, torch.ones_like(kept))
         assert tangent(_attend, (cos, sin)) is not None
         p["up"] = kept
+
+
+@pytest.mark.parametrize("tokens", [1, 37])
+@torch.no_grad()
+def test_rope_tables_of_other_forms(tokens):
+    """Tables that broadcast over rows or tokens and tables of 16-bit floats
+    give what their expanded float32 form gives; float64 tables and tables of
+    other shapes run the torch operations."""
+    model, x, _ = _small_model(tokens)
+    cos, sin = model.rope(torch.arange(tokens, device=DEV)[None] + 3)
+    run = lambda c, s: model.layer(0, x, _attend, (c, s))  # noqa: E731
+    expand = lambda *tables: tuple(t.float().expand(2, tokens, 64).contiguous() for t in tables)  # noqa: E731
+    want = run(*expand(cos, sin))
+    assert torch.equal(run(cos, sin), want)
+    assert torch.equal(run(cos.expand(2, tokens, 64), sin), want)
+    top, states = model.layers_forward(x, lambda i, q: _attend(q), (cos, sin))
+    assert torch.equal(states[1], want)
+    for one in (cos[:, :1], cos[:, :1].expand(2, 1, 64), cos[:, :, :1]):
+        assert torch.equal(run(one, sin), run(*expand(one, sin)))
+    for dtype in (torch.bfloat16, torch.float16):
+        c, s = cos.to(dtype), sin.to(dtype)
+        assert torch.equal(run(c, s), run(*expand(c, s)))
+        assert torch.equal(run(c, sin), run(*expand(c, sin)))
+    for c, s in ((cos.double(), sin.double()), (cos[0, :1], sin[0, :1])):
+        with torch.enable_grad():
+            eager = run(c, s)
+        assert torch.equal(run(c, s), eager)

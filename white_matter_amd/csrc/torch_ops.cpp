@@ -989,26 +989,42 @@ Tensor residual_norm(const Tensor& x, const c10::optional<Tensor>& delta, const 
   return normed;
 }
 
-// The checked RoPE tables of tokens x (B, T, ...): c and s are cos and sin
-// with one pair of row strides and 16-byte aligned rows.
-void rope_rows(const Tensor& cos, const Tensor& sin, const Tensor& weight, const Tensor& x, int64_t dim, Tensor& c, Tensor& s) {
-  TORCH_CHECK_VALUE(cos.dim() == 3 && cos.size(0) == x.size(0) && cos.size(1) == x.size(1) && cos.size(2) == dim &&
-                        sin.sizes() == cos.sizes() && cos.scalar_type() == at::kFloat && sin.scalar_type() == at::kFloat &&
-                        weight.dim() == 1 && weight.size(0) == dim && cos.device() == x.device() &&
-                        sin.device() == x.device() && weight.device() == x.device(),
-                    "cos and sin must be float32 (B, T, D) and weight (D,) on the queries' device");
+// Contiguous and 16-byte aligned.
+Tensor dense16(const Tensor& t) {
+  Tensor c = t.contiguous();
+  return reinterpret_cast<uintptr_t>(c.data_ptr()) % 16 ? c.clone() : c;
+}
+
+// The checked RoPE tables of tokens x (B, T, ...): c and s are cos and sin,
+// expanded over rows and tokens, as float32 with 16-byte aligned rows (16-bit
+// tables are exact in it) and one pair of row strides, `strides`.
+void rope_rows(const Tensor& cos, const Tensor& sin, const Tensor& weight, const Tensor& x, int64_t dim, Tensor& c, Tensor& s,
+               int64_t (&strides)[2]) {
+  const int64_t want[3] = {x.size(0), x.size(1), dim};
+  for (const Tensor* t : {&cos, &sin}) {
+    const auto type = t->scalar_type();
+    bool ok = t->dim() == 3 && t->device() == x.device() && (type == at::kFloat || type == at::kBFloat16 || type == at::kHalf);
+    for (int d = 0; ok && d < 3; ++d) ok = t->size(d) == want[d] || t->size(d) == 1;
+    TORCH_CHECK_VALUE(ok, "cos and sin must be float32 or 16-bit tables that expand to (B, T, D), on the queries' device");
+  }
+  TORCH_CHECK_VALUE(weight.dim() == 1 && weight.size(0) == dim && weight.device() == x.device(),
+                    "weight must be (D,) on the queries' device");
   c10::OptionalDeviceGuard guard(x.device());
-  auto rows = [](const Tensor& t) {
-    const bool ok = t.stride(-1) == 1 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 && t.stride(0) % 4 == 0 &&
-                    t.stride(1) % 4 == 0;
-    return ok ? t : t.contiguous().clone();
+  auto step = [](const Tensor& t, int d) { return t.size(d) > 1 ? t.stride(d) : 0; };
+  auto rows = [&](const Tensor& t) {
+    const Tensor e = t.to(at::kFloat).expand(want);
+    const bool ok = e.stride(-1) == 1 && reinterpret_cast<uintptr_t>(e.data_ptr()) % 16 == 0 && step(e, 0) % 4 == 0 &&
+                    step(e, 1) % 4 == 0;
+    return ok ? e : dense16(e);
   };
   c = rows(cos);
   s = rows(sin);
-  if (c.strides() != s.strides()) {
-    c = cos.contiguous().clone();
-    s = sin.contiguous().clone();
+  if (step(c, 0) != step(s, 0) || step(c, 1) != step(s, 1)) {
+    c = dense16(c);
+    s = dense16(s);
   }
+  strides[0] = step(c, 0);
+  strides[1] = step(c, 1);
 }
 
 // Queries (B, T, H * D) bf16 -> (B, T, H, D): rms_norm, weight, bf16, RoPE with
@@ -1017,23 +1033,21 @@ Tensor query_norm_rope(const Tensor& q, const Tensor& weight, const Tensor& cos,
   TORCH_CHECK_VALUE(q.dim() == 3 && q.scalar_type() == at::kBFloat16 && heads > 0 && q.size(2) % heads == 0,
                     "query_norm_rope takes bfloat16 (B, T, H * D) queries");
   const int64_t dim = q.size(2) / heads;
+  wmx_query_rope_args a;
+  std::memset(&a, 0, sizeof(a));
   Tensor c, s;
-  rope_rows(cos, sin, weight, q, dim, c, s);
+  rope_rows(cos, sin, weight, q, dim, c, s, a.rope_stride);
   c10::OptionalDeviceGuard guard(q.device());
   Tensor x = q.contiguous(), w = weight.contiguous();
   if (reinterpret_cast<uintptr_t>(x.data_ptr()) % 16) x = x.clone();
   if (reinterpret_cast<uintptr_t>(w.data_ptr()) % 16) w = w.clone();
   Tensor out = at::empty({q.size(0), q.size(1), heads, dim}, q.options());
-  wmx_query_rope_args a;
-  std::memset(&a, 0, sizeof(a));
   a.q = x.data_ptr();
   a.weight = w.data_ptr();
   a.weight_dtype = float_dtype(w, "weight");
   a.cos = c.data_ptr<float>();
   a.sin = s.data_ptr<float>();
   a.out = out.data_ptr();
-  a.rope_stride[0] = c.stride(0);
-  a.rope_stride[1] = c.stride(1);
   a.tokens = q.size(0) * q.size(1);
   a.tokens_per_row = std::max<int64_t>(q.size(1), 1);
   a.heads = (int32_t)heads;
@@ -1054,12 +1068,6 @@ Tensor silu_mul(const Tensor& gate, const Tensor& up) {
   Tensor out = at::empty(gate.sizes(), gate.options());
   check_rc(wmx_silu_mul(g.data_ptr(), u.data_ptr(), out.data_ptr(), gate.numel(), stream_of(gate)), "wmx_silu_mul");
   return out;
-}
-
-// Contiguous and 16-byte aligned.
-Tensor dense16(const Tensor& t) {
-  Tensor c = t.contiguous();
-  return reinterpret_cast<uintptr_t>(c.data_ptr()) % 16 ? c.clone() : c;
 }
 
 // Products of bf16 rows x (..., in) with (out, in) weights (linear.hip): the
@@ -1148,7 +1156,8 @@ Tensor linear_query(const Tensor& x, const Tensor& weight, const Tensor& norm, c
   TORCH_CHECK_VALUE(x.dim() == 3 && heads > 0 && weight.size(0) % heads == 0, "queries take rows (B, T, in) and a (H * D, in) weight");
   const int64_t dim = weight.size(0) / heads;
   Tensor c, s;
-  rope_rows(cos, sin, norm, x, dim, c, s);
+  int64_t rope_stride[2];
+  rope_rows(cos, sin, norm, x, dim, c, s, rope_stride);
   c10::OptionalDeviceGuard guard(x.device());
   const Tensor rows = dense16(x), w = dense16(weight), n = dense16(norm);
   Tensor out = at::empty({x.size(0), x.size(1), heads, dim}, x.options());
@@ -1160,8 +1169,8 @@ Tensor linear_query(const Tensor& x, const Tensor& weight, const Tensor& norm, c
   a.eps = (float)eps;
   a.cos = c.data_ptr<float>();
   a.sin = s.data_ptr<float>();
-  a.rope_stride[0] = c.stride(0);
-  a.rope_stride[1] = c.stride(1);
+  a.rope_stride[0] = rope_stride[0];
+  a.rope_stride[1] = rope_stride[1];
   a.tokens_per_row = std::max<int64_t>(x.size(1), 1);
   check_rc(wmx_linear(&a, stream_of(x)), "wmx_linear");
   return out;

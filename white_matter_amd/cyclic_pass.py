@@ -91,6 +91,10 @@ _GATED_TILES = 768
 _POOL_TILES = 1024
 
 
+# RoPE tables that the kernels take (float64 ones are not exact in fp32)
+_ROPE_DTYPES = (torch.float32, torch.bfloat16, torch.float16)
+
+
 def _tiles(rows: int, features: int) -> int:
     return (rows + 63) // 64 * ((features + 63) // 64)
 
@@ -245,16 +249,22 @@ class FeedbackModel:
         x = F.rms_norm(x.to(self.residual_dtype), (x.shape[-1],), None, eps)
         return (x * weight.to(self.residual_dtype)).to(self.dtype)
 
-    def _fused(self, x: torch.Tensor) -> bool:
+    def _fused(self, x: torch.Tensor, rope=()) -> bool:
         """The layer's token-local steps run as HIP kernels: on the GPU without
         gradients (forward-mode ones included) and vmap, bf16 activations over an
-        fp32 residual stream, in the sizes that the kernels take. Other calls run
-        the torch operations."""
+        fp32 residual stream, in the sizes that the kernels take, with RoPE tables
+        of up to 32 bits that expand to (B, T, D). Other calls run the torch
+        operations."""
         c = self.config
         return (
             x.is_cuda and x.dtype == self.residual_dtype == torch.float32 and self.dtype == torch.bfloat16
             and not torch.is_grad_enabled() and not _kernels.transformed() and c.head_dim in (64, 96, 128)
             and c.hidden_size % 8 == 0 and c.hidden_size <= 4096 and c.intermediate_size % 8 == 0
+            and all(
+                t.dtype in _ROPE_DTYPES and t.ndim == 3
+                and all(n in (1, m) for n, m in zip(t.shape, (*x.shape[:2], c.head_dim)))
+                for t in rope
+            )
         )
 
     def _layer_fused(self, index: int, h: torch.Tensor, x: torch.Tensor, out: torch.Tensor, attend, rope) -> torch.Tensor:
@@ -284,7 +294,7 @@ class FeedbackModel:
         """decoder_layer.py:51-72 with layers/white_matter.py:109-116, 199:
         x (B, T, d) residual; attend(q (B, Hq, T, D)) -> (B, T, Hq, D)."""
         c, p = self.config, self.layers[index]
-        if self._fused(x):
+        if self._fused(x, rope):
             ops = torch.ops.white_matter
             h = ops.residual_norm(x, None, None, p["input_norm"], c.rms_norm_eps)
             mid, out = (torch.empty(x.shape, device=x.device, dtype=x.dtype) for _ in range(2))
@@ -305,7 +315,7 @@ class FeedbackModel:
     def layers_forward(self, x: torch.Tensor, attend_layer, rope) -> tuple[torch.Tensor, list[torch.Tensor]]:
         """run_feedback_layers (decoder_layer.py:75-94) with the top output kept:
         returns the output and the L + 1 pool sources."""
-        if self._fused(x):
+        if self._fused(x, rope):
             x, stacked = self.layers_stacked(x, attend_layer, rope)
             return x, list(stacked.unbind(2))
         states = []
@@ -319,7 +329,7 @@ class FeedbackModel:
         """`layers_forward` with the L + 1 pool sources as one (B, T, L + 1, d)
         tensor. On the GPU the residual stream lives in it: each layer's last
         add, with the next layer's norm, writes the next source."""
-        if not self._fused(x):
+        if not self._fused(x, rope):
             x, states = self.layers_forward(x, attend_layer, rope)
             return x, torch.stack(states, dim=2)
         c, ops, eps = self.config, torch.ops.white_matter, self.config.rms_norm_eps
