@@ -265,3 +265,23 @@ def test_rope_tables_of_other_forms(tokens):
         with torch.enable_grad():
             eager = run(c, s)
         assert torch.equal(run(c, s), eager)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float64])
+@torch.no_grad()
+def test_norm_weights_of_other_types(dtype):
+    """Norm weights are read in float32, as the torch operations cast them."""
+    model, x, _ = _small_model(9)
+    rope = model.rope(torch.arange(9, device=DEV).expand(2, 9))
+    run = lambda: (model.layer(0, x, _attend, rope), *model.layers_forward(x, lambda i, q: _attend(q), rope)[1], model.logits(x))  # noqa: E731
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    weights = {n: (1 + 0.1 * torch.randn(model.layers[0][n].shape, generator=gen, device=DEV)).to(dtype)
+               for n in ("input_norm", "q_norm", "post_norm")}
+    results = []
+    for cast in (dtype, torch.float32):
+        for p in model.layers:
+            p.update({n: w.to(cast) for n, w in weights.items()})
+        model.final_norm = weights["input_norm"].to(cast)
+        results.append(run())
+    for got, want in zip(*results, strict=True):
+        assert torch.equal(got, want)

@@ -921,10 +921,17 @@ void strict_decode_out(const Tensor& out, const Tensor& query, const Tensor& key
 }
 
 // ------------------------------------------------- layer steps ----
-int32_t float_dtype(const Tensor& t, const char* what) {
-  TORCH_CHECK_TYPE(t.scalar_type() == at::kFloat || t.scalar_type() == at::kBFloat16, what, " must be float32 or bfloat16");
-  return t.scalar_type() == at::kFloat ? WMX_DTYPE_F32 : WMX_DTYPE_BF16;
+// Contiguous and 16-byte aligned.
+Tensor dense16(const Tensor& t) {
+  Tensor c = t.contiguous();
+  return reinterpret_cast<uintptr_t>(c.data_ptr()) % 16 ? c.clone() : c;
 }
+
+// A norm's weight as the kernels read it: bfloat16, or float32 (the type that
+// the norm's arithmetic casts any other to).
+Tensor norm_weight(const Tensor& t) { return dense16(t.scalar_type() == at::kBFloat16 ? t : t.to(at::kFloat)); }
+
+int32_t float_dtype(const Tensor& t) { return t.scalar_type() == at::kFloat ? WMX_DTYPE_F32 : WMX_DTYPE_BF16; }
 
 // The row stride of a (..., hidden) fp32 tensor whose rows are equally spaced.
 bool row_stride(const Tensor& t, int64_t& stride) {
@@ -977,22 +984,15 @@ Tensor residual_norm(const Tensor& x, const c10::optional<Tensor>& delta, const 
   if (weight) {
     TORCH_CHECK_VALUE(weight->dim() == 1 && weight->size(0) == hidden && weight->device() == x.device(),
                       "weight must be (hidden,)");
-    w = weight->contiguous();
-    if (reinterpret_cast<uintptr_t>(w.data_ptr()) % 16) w = w.clone();
+    w = norm_weight(*weight);
     a.weight = w.data_ptr();
-    a.weight_dtype = float_dtype(w, "weight");
+    a.weight_dtype = float_dtype(w);
     a.normed = normed.data_ptr();
   } else {
     a.weight_dtype = WMX_DTYPE_F32;
   }
   check_rc(wmx_residual_norm(&a, stream_of(x)), "wmx_residual_norm");
   return normed;
-}
-
-// Contiguous and 16-byte aligned.
-Tensor dense16(const Tensor& t) {
-  Tensor c = t.contiguous();
-  return reinterpret_cast<uintptr_t>(c.data_ptr()) % 16 ? c.clone() : c;
 }
 
 // The checked RoPE tables of tokens x (B, T, ...): c and s are cos and sin,
@@ -1038,13 +1038,11 @@ Tensor query_norm_rope(const Tensor& q, const Tensor& weight, const Tensor& cos,
   Tensor c, s;
   rope_rows(cos, sin, weight, q, dim, c, s, a.rope_stride);
   c10::OptionalDeviceGuard guard(q.device());
-  Tensor x = q.contiguous(), w = weight.contiguous();
-  if (reinterpret_cast<uintptr_t>(x.data_ptr()) % 16) x = x.clone();
-  if (reinterpret_cast<uintptr_t>(w.data_ptr()) % 16) w = w.clone();
+  const Tensor x = dense16(q), w = norm_weight(weight);
   Tensor out = at::empty({q.size(0), q.size(1), heads, dim}, q.options());
   a.q = x.data_ptr();
   a.weight = w.data_ptr();
-  a.weight_dtype = float_dtype(w, "weight");
+  a.weight_dtype = float_dtype(w);
   a.cos = c.data_ptr<float>();
   a.sin = s.data_ptr<float>();
   a.out = out.data_ptr();
@@ -1159,13 +1157,13 @@ Tensor linear_query(const Tensor& x, const Tensor& weight, const Tensor& norm, c
   int64_t rope_stride[2];
   rope_rows(cos, sin, norm, x, dim, c, s, rope_stride);
   c10::OptionalDeviceGuard guard(x.device());
-  const Tensor rows = dense16(x), w = dense16(weight), n = dense16(norm);
+  const Tensor rows = dense16(x), w = dense16(weight), n = norm_weight(norm);
   Tensor out = at::empty({x.size(0), x.size(1), heads, dim}, x.options());
   wmx_linear_args a;
   linear_args(a, rows, w, out, WMX_LINEAR_QUERY);
   a.head_dim = (int32_t)dim;
   a.norm = n.data_ptr();
-  a.norm_dtype = float_dtype(n, "weight");
+  a.norm_dtype = float_dtype(n);
   a.eps = (float)eps;
   a.cos = c.data_ptr<float>();
   a.sin = s.data_ptr<float>();
