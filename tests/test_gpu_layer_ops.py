@@ -285,3 +285,21 @@ def test_norm_weights_of_other_types(dtype):
         results.append(run())
     for got, want in zip(*results, strict=True):
         assert torch.equal(got, want)
+
+
+def test_autocast_to_another_type():
+    """Under autocast to float16 the products round to float16, as with
+    gradients on; under autocast to the model's own type nothing changes."""
+    model, x, _ = _small_model(9)
+    rope = model.rope(torch.arange(9, device=DEV).expand(2, 9))
+    run = lambda: (model.layer(0, x, _attend, rope), model.logits(x))  # noqa: E731
+    with torch.autocast("cuda", torch.float16):
+        want = run()
+        with torch.no_grad():
+            got = run()
+    assert all(torch.equal(g, w) and g.dtype == w.dtype for g, w in zip(got, want, strict=True))
+    with torch.no_grad():
+        plain = run()
+        with torch.autocast("cuda", torch.bfloat16):
+            same = run()
+    assert all(torch.equal(g, w) and g.dtype == w.dtype for g, w in zip(same, plain, strict=True))

@@ -254,12 +254,14 @@ class FeedbackModel:
         gradients (forward-mode ones included) and vmap, bf16 activations over an
         fp32 residual stream, in the sizes that the kernels take, with RoPE tables
         of up to 32 bits that expand to (B, T, D). Other calls run the torch
-        operations."""
+        operations, and so does autocast to another type, which the kernels do not
+        follow."""
         c = self.config
         return (
             x.is_cuda and x.dtype == self.residual_dtype == torch.float32 and self.dtype == torch.bfloat16
             and not torch.is_grad_enabled() and not _kernels.transformed() and c.head_dim in (64, 96, 128)
             and c.hidden_size % 8 == 0 and c.hidden_size <= 4096 and c.intermediate_size % 8 == 0
+            and not (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != self.dtype)
             and all(
                 t.dtype in _ROPE_DTYPES and t.ndim == 3
                 and all(n in (1, m) for n, m in zip(t.shape, (*x.shape[:2], c.head_dim)))
