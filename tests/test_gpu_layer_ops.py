@@ -303,3 +303,17 @@ def test_autocast_to_another_type():
         with torch.autocast("cuda", torch.bfloat16):
             same = run()
     assert all(torch.equal(g, w) and g.dtype == w.dtype for g, w in zip(same, plain, strict=True))
+
+
+@torch.no_grad()
+def test_layer_outputs_own_their_memory():
+    """The top output and the sources are contiguous tensors of their own: a
+    caller may view them flat, and keeping one does not keep the others."""
+    model, x, _ = _small_model(9)
+    rope = model.rope(torch.arange(9, device=DEV).expand(2, 9))
+    top, states = model.layers_forward(x, lambda i, q: _attend(q), rope)
+    assert states[0] is x and top is states[-1] and len(states) == 3
+    for t in states:
+        assert t.view(-1, 136).shape == (18, 136) and t.untyped_storage().nbytes() == t.numel() * 4
+    stacked = model.layers_stacked(x, lambda i, q: _attend(q), rope)
+    assert torch.equal(stacked[0], top) and torch.equal(stacked[1], torch.stack(states, 2))

@@ -317,9 +317,6 @@ class FeedbackModel:
     def layers_forward(self, x: torch.Tensor, attend_layer, rope) -> tuple[torch.Tensor, list[torch.Tensor]]:
         """run_feedback_layers (decoder_layer.py:75-94) with the top output kept:
         returns the output and the L + 1 pool sources."""
-        if self._fused(x, rope):
-            x, stacked = self.layers_stacked(x, attend_layer, rope)
-            return x, list(stacked.unbind(2))
         states = []
         for index in range(self.config.num_layers):
             states.append(x)
