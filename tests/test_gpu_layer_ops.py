@@ -317,3 +317,27 @@ def test_layer_outputs_own_their_memory():
         assert t.view(-1, 136).shape == (18, 136) and t.untyped_storage().nbytes() == t.numel() * 4
     stacked = model.layers_stacked(x, lambda i, q: _attend(q), rope)
     assert torch.equal(stacked[0], top) and torch.equal(stacked[1], torch.stack(states, 2))
+
+
+@torch.no_grad()
+def test_a_subclass_keeps_its_own_layers():
+    """A model that redefines a layer, or how the layers follow each other,
+    gets its own in the pass too."""
+
+    class OwnLayer(FeedbackModel):
+        def layer(self, index, x, attend, rope):
+            return super().layer(index, x, attend, rope) + 1
+
+    class OwnLayers(FeedbackModel):
+        def layers_forward(self, x, attend_layer, rope):
+            return x * 2, [x] * self.config.num_sources
+
+    plain, x, _ = _small_model(9)
+    rope = plain.rope(torch.arange(9, device=DEV).expand(2, 9))
+    for kind in (OwnLayer, OwnLayers):
+        model = kind(plain.config, device=DEV, seed=5)
+        top, states = model.layers_forward(x, lambda i, q: _attend(q), rope)
+        got = model.layers_stacked(x, lambda i, q: _attend(q), rope)
+        assert torch.equal(got[0], top) and torch.equal(got[1], torch.stack(states, 2))
+    plain.layer = lambda index, x, attend, rope: x + 1
+    assert torch.equal(plain.layers_stacked(x, lambda i, q: _attend(q), rope)[0], x + 1 + 1)

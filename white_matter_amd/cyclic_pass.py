@@ -327,8 +327,13 @@ class FeedbackModel:
     def layers_stacked(self, x: torch.Tensor, attend_layer, rope) -> tuple[torch.Tensor, torch.Tensor]:
         """`layers_forward` with the L + 1 pool sources as one (B, T, L + 1, d)
         tensor. On the GPU the residual stream lives in it: each layer's last
-        add, with the next layer's norm, writes the next source."""
-        if not self._fused(x, rope):
+        add, with the next layer's norm, writes the next source. A model that
+        redefines `layer` or `layers_forward` runs its own."""
+        own = any(
+            getattr(getattr(self, name), "__func__", None) is not getattr(FeedbackModel, name)
+            for name in ("layer", "layers_forward")
+        )
+        if own or not self._fused(x, rope):
             x, states = self.layers_forward(x, attend_layer, rope)
             return x, torch.stack(states, dim=2)
         c, ops, eps = self.config, torch.ops.white_matter, self.config.rms_norm_eps
