@@ -332,6 +332,24 @@ def test_producer_backward_kernels(batch, tokens, sources, hidden, channels, str
         assert ours <= 1.1 * theirs + 2**-9, f"input {n}: rel-L2 {ours:.3e}, the eager steps' {theirs:.3e}"
 
 
+def test_producer_batched_gradients():
+    """A vmapped backward (is_grads_batched) through the training form: each
+    batch entry within the training form's bar of its own backward."""
+    stacked, pre_mix, router, gain = _producer_inputs(2, 4, 5, 64, 3, 45, torch.float32, torch.float32)
+    flat = [stacked, pre_mix[0], pre_mix[1], *router[0], *router[1], gain[0], gain[1]]
+    leaves = [t.to(DEV).clone().requires_grad_() for t in flat]
+    outs = kv_pool.projection_inputs(leaves[0], (leaves[1], leaves[2]), ((leaves[3], leaves[4]), (leaves[5], leaves[6])),
+                                     (leaves[7], leaves[8]))
+    gen = torch.Generator().manual_seed(11)
+    probes = [torch.randn(3, *o.shape, generator=gen).bfloat16().to(DEV) for o in outs]
+    batched = torch.autograd.grad(outs, leaves, probes, is_grads_batched=True, retain_graph=True)
+    for i in range(3):
+        one = torch.autograd.grad(outs, leaves, [p[i] for p in probes], retain_graph=True)
+        for n, (b, g) in enumerate(zip(batched, one, strict=True)):
+            assert b[i].shape == g.shape and b.dtype == g.dtype
+            assert (b[i] - g).norm() <= 2e-2 * g.norm(), f"input {n}, entry {i}"
+
+
 def test_producer_rejects_bad_shapes():
     stacked, pre_mix, router, gain = _producer_inputs(1, 2, 3, 64, 2, 0, torch.float32, torch.float32)
     args = (tuple(pre_mix.to(DEV)), tuple((w.to(DEV), b.to(DEV)) for w, b in router), tuple(gain.to(DEV)))

@@ -31,14 +31,18 @@ def guard_capture(what: str) -> None:
         )
 
 
-def transformed() -> bool:
-    """Whether the caller runs under a functorch transform (vmap, jvp, the
-    batched backward of is_grads_batched) or inside a forward-mode dual level.
-    Disabling gradients disables neither, and any tensor of the call (an input,
-    a weight, what a callback returns) may be batched or carry a tangent there:
-    operators without a rule for them would refuse it or drop the tangent, so
-    the torch operations run."""
-    return torch._C._are_functorch_transforms_active() or forward_ad._current_level >= 0
+def transformed(*grads: torch.Tensor) -> bool:
+    """Whether the caller runs under a functorch transform (vmap, jvp) or inside
+    a forward-mode dual level, or a gradient that it got is batched
+    (torch.autograd.grad's is_grads_batched, a vmap of its own). Disabling
+    gradients disables none, and any tensor of the call (an input, a weight, what
+    a callback returns) may be batched or carry a tangent there: operators without
+    a rule for them would refuse it or drop the tangent, so the torch operations
+    run."""
+    if torch._C._are_functorch_transforms_active() or forward_ad._current_level >= 0:
+        return True
+    # (traced gradients are not batched)
+    return not torch.compiler.is_compiling() and any(torch._C._functorch.is_legacy_batchedtensor(g) for g in grads)
 
 
 def kernel_head_dim(dim: int) -> int | None:

@@ -34,7 +34,7 @@ from __future__ import annotations
 import torch
 import torch.nn.functional as F
 
-from . import _native
+from . import _kernels, _native
 
 _DTYPES = {torch.float32: _native.DTYPE_F32, torch.bfloat16: _native.DTYPE_BF16}
 
@@ -441,10 +441,10 @@ def _producer_bwd_fits(sources: int, hidden: int, channels: int) -> bool:
 
 class _ProjectionInputsFn(torch.autograd.Function):
     """Training form: HIP kernels forward and backward (wmx_kv_mix_bwd, from
-    the saved inputs and logits). Sizes that the backward kernels do not take
-    recompute the reference's eager steps from the saved inputs and
-    differentiate them (the reference trains _project under selective
-    checkpointing with the same recompute)."""
+    the saved inputs and logits). Sizes that the backward kernels do not take,
+    and backwards under a transform, recompute the reference's eager steps from
+    the saved inputs and differentiate them (the reference trains _project under
+    selective checkpointing with the same recompute)."""
 
     @staticmethod
     def forward(ctx, stacked, pre_k, pre_v, w_k, b_k, w_v, b_v, gain_k, gain_v, eps, mix_eps, stride):
@@ -460,10 +460,10 @@ class _ProjectionInputsFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_k, grad_v):
-        saved = ctx.saved_tensors
+        *saved, alpha = ctx.saved_tensors if ctx.on_device else (*ctx.saved_tensors, None)
         eps, mix_eps, stride = ctx.config
-        if ctx.on_device:
-            stacked, pre_k, pre_v, w_k, b_k, w_v, b_v, gain_k, gain_v, alpha = saved
+        if ctx.on_device and not _kernels.transformed(grad_k, grad_v):
+            stacked, pre_k, pre_v, w_k, _, w_v, _, gain_k, gain_v = saved
             with torch.no_grad():
                 grads = torch.ops.white_matter.kv_producer_bwd(
                     stacked, pre_k, pre_v, w_k, w_v, gain_k, gain_v, alpha, grad_k, grad_v, eps, mix_eps, stride
