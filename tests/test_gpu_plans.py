@@ -116,3 +116,18 @@ def test_plans_take_the_device_path():
     ids = torch.cat((torch.full((2, 1), -1, device=DEV), docs), 1)
     cyc = prepare_cyclic_attention_metadata(docs[:, ::4].contiguous(), ids)
     assert _plans.cyclic_plan(tuple(cyc), 128, 513, 4, 0, 64, 96)[0][0] == 2
+
+
+@torch.no_grad()
+def test_schedules_without_keys_or_queries():
+    """Segments without keys give zeros, and a schedule without queries or keys
+    is planned as on the host (an empty tensor's address reads as missing)."""
+    ints = lambda *v: torch.tensor(v, device=DEV, dtype=torch.int32)  # noqa: E731
+    none = torch.empty(0, device=DEV, dtype=torch.int64)
+    rows = torch.tensor([0, 1, 2, 5, 6], device=DEV)
+    metadata = strict.StrictCausalMetadata(rows, none, ints(0, 3, 5), ints(0, 0, 0), 4, 6, 6)
+    _compare_packed(metadata, 2, 4, 6, "no keys")
+    _compare_packed(strict.StrictCausalMetadata(none, torch.arange(3, device=DEV), ints(0, 0), ints(0, 3), 4, 6, 6), 2, 4, 6, "no queries")
+    _compare_packed(strict.StrictCausalMetadata(none, none, ints(0, 0), ints(0, 0), 4, 6, 6), 2, 4, 6, "neither")
+    q, k, v = (torch.randn(2, 2, n, 64, device=DEV).bfloat16() for n in (4, 6, 6))
+    assert not strict.strict_causal_attention(q, k, v, metadata=metadata).any()

@@ -120,6 +120,8 @@ def packed_plan(
     schedule itself) and the work lists."""
     device = schedule[0].device
     segments = schedule[2].numel() - 1
+    if schedule[0].numel() == 0 or schedule[1].numel() == 0:
+        return None  # (an empty tensor's address is null, which reads as missing)
     if segments < 1 or segments > _MAX_SEGMENTS or schedule[3].numel() != segments + 1 or max(length, key_slots) > _MAX_COUNT:
         return None
     a = _native.PlanArgs()
