@@ -19,7 +19,7 @@ import torch.nn.functional as F
 
 from oracle import kv_pool as ref
 from tests.numerics import assert_bf16_close
-from white_matter_amd import kv_pool
+from white_matter_amd import _native, kv_pool
 from white_matter_amd.cyclic_pass import FeedbackConfig, FeedbackModel, HipKernels
 
 pytestmark = pytest.mark.gpu
@@ -348,6 +348,46 @@ def test_producer_batched_gradients():
         for n, (b, g) in enumerate(zip(batched, one, strict=True)):
             assert b[i].shape == g.shape and b.dtype == g.dtype
             assert (b[i] - g).norm() <= 2e-2 * g.norm(), f"input {n}, entry {i}"
+
+
+def test_producer_backward_reads_a_part_of_the_sources():
+    """A router that reads fewer sources than its stride would reach: the same
+    gradients as one that reads them all with zero weights for the others. (The
+    Python operator always reads to the last source; a C caller need not.)"""
+    batch, tokens, sources, hidden, channels, read = 2, 9, 9, 128, 3, 4
+    gen = torch.Generator().manual_seed(9)
+    rand = lambda *shape: torch.randn(*shape, generator=gen).bfloat16().to(DEV)  # noqa: E731
+    x, pre, gain = rand(batch, tokens, sources, hidden), rand(2, sources, hidden), rand(2, channels, hidden)
+    premixed = kv_pool.kv_premix(x, pre[0], pre[1], 1e-6)
+    alpha, grad = rand(2, batch * tokens, channels * sources), rand(2, channels, batch * tokens, hidden)
+    part = rand(2, channels * sources, read * hidden)
+    whole = torch.zeros(2, channels * sources, sources * hidden, device=DEV, dtype=torch.bfloat16)
+    whole[..., : read * hidden] = part
+    results = []
+    for weight, count in ((part, read), (whole, sources)):
+        a = _native.KvMixBwdArgs()
+        out = dict(
+            sources=torch.empty_like(x), pre_mix=torch.empty_like(pre), gain=torch.empty_like(gain),
+            bias=torch.empty(2, channels * sources, device=DEV, dtype=torch.bfloat16), weight=torch.empty_like(weight),
+        )
+        a.sources, a.source_stride, a.grad_sources = x.data_ptr(), x.stride()[:3], out["sources"].data_ptr()
+        a.source_dtype = a.weight_dtype = a.grad_weight_dtype = _native.DTYPE_BF16
+        a.batch, a.tokens, a.num_sources, a.hidden, a.channels = batch, tokens, sources, hidden, channels
+        a.read_start, a.read_stride, a.read_sources = 0, 1, count
+        a.eps, a.mix_eps, a.alpha_stride = 1e-6, 1e-4, channels * sources
+        for side in range(2):
+            a.premixed[side], a.alpha[side], a.grad[side] = (t[side].data_ptr() for t in (premixed, alpha, grad))
+            a.pre_mix[side], a.gain[side], a.weight[side] = (t[side].data_ptr() for t in (pre, gain, weight))
+            a.grad_pre_mix[side], a.grad_gain[side] = out["pre_mix"][side].data_ptr(), out["gain"][side].data_ptr()
+            a.grad_bias[side], a.grad_weight[side] = out["bias"][side].data_ptr(), out["weight"][side].data_ptr()
+        workspace = torch.empty(_native.kv_mix_bwd_workspace_size(a), device=DEV, dtype=torch.uint8)
+        a.workspace, a.workspace_bytes = workspace.data_ptr(), workspace.numel()
+        _native.kv_mix_bwd(a, x.device)
+        results.append(out)
+    part, whole = results
+    assert torch.equal(part.pop("weight"), whole.pop("weight")[..., : read * hidden].contiguous())
+    for name, g in part.items():
+        assert torch.equal(g, whole[name]), name
 
 
 def test_producer_rejects_bad_shapes():

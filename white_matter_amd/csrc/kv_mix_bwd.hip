@@ -435,7 +435,8 @@ __global__ __launch_bounds__(256, VPT * CM <= 8 ? 2 : 1) void sources_bwd_kernel
   for (int g = 0; g < G; ++g) {
     src_at[g] = min(s0 + g, S - 1);
     const int rel = src_at[g] - a.read_start;
-    read_at[g] = rel >= 0 && rel % a.read_stride == 0 ? rel / a.read_stride : -1;
+    const bool read = rel >= 0 && rel % a.read_stride == 0 && rel / a.read_stride < a.read_sources;
+    read_at[g] = read ? rel / a.read_stride : -1;
 #pragma unroll
     for (int side = 0; side < 2; ++side)
 #pragma unroll
