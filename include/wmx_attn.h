@@ -647,7 +647,8 @@ typedef struct wmx_pool_project_args {
  * entries of WMX_UNIT_FIELDS ints, heaviest first; segments of 1 to
  * fused_rows queries with a key also form f_units, and bq_units / bk_units
  * are q_units / k_units without them (fused_rows 0: all three NULL).
- * total_segments < 2^20, key tiles and query tiles of a segment < 2^15.
+ * q_len, k_len and units of a list < 2^21, batch * q_len and batch * k_len
+ * < 2^31, total_segments < 2^20.
  */
 enum {
   WMX_PLAN_QUERIES = 0,      /* queries of segments */

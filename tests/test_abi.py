@@ -203,3 +203,26 @@ def test_fused_segment_list_checks():
     a.f_units, a.query_indices = 0x1000, None
     assert lib.wmx_attn_bwd(ctypes.byref(a), None) == -1
     assert b"varlen schedule" in lib.wmx_last_error()
+
+
+def test_plan_size_checks():
+    """Rows, keys and units past what the plan kernels' scans count in one word
+    (21 bits), and row indices past 32 bits, are refused before a launch."""
+    lib = _native.load()
+    args = lambda: _native.PlanArgs(  # noqa: E731
+        q_seg=0x1000, k_seg=0x1000, q_start=0x1000, k_qend=0x1000, counts=0x1000, workspace=0x1000, workspace_bytes=1 << 60,
+        unit_workspace=0x1000, unit_workspace_bytes=1 << 60, out_query_indices=0x1000, out_key_indices=0x1000,
+        out_cu_queries=0x1000, out_cu_keys=0x1000, ds_offsets=0x1000, q_units=0x1000, k_units=0x1000, batch=1, q_len=8, k_len=8,
+        query_stride=1, key_tile=64, total_segments=1,
+    )
+    for field in ("q_len", "k_len"):
+        for value, batch in ((1 << 21, 1), ((1 << 21) - 1, 1 << 11)):
+            a = args()
+            setattr(a, field, value)
+            a.batch = batch
+            for entry in (lib.wmx_plan_count, lib.wmx_plan_fill):
+                assert entry(ctypes.byref(a), None) == -2 and b"2^21" in lib.wmx_last_error()
+    for field in ("num_q_units", "num_k_units", "num_f_units"):
+        a = args()
+        setattr(a, field, 1 << 21)
+        assert lib.wmx_plan_fill(ctypes.byref(a), None) == -2 and b"units" in lib.wmx_last_error()

@@ -81,7 +81,7 @@ def cyclic_plan(
     facts of `_cyclic_schedule` and its tensors."""
     device = meta[0].device
     batch = meta[0].shape[0]
-    if max(q_len, k_len) > _MAX_COUNT:
+    if max(q_len, k_len) > _MAX_COUNT or batch * max(q_len, k_len) >= 2**31:
         return None
     a = _native.PlanArgs()
     a.q_seg, a.k_seg, a.q_start, a.k_qend = (t.data_ptr() for t in meta)
@@ -122,7 +122,9 @@ def packed_plan(
     segments = schedule[2].numel() - 1
     if schedule[0].numel() == 0 or schedule[1].numel() == 0:
         return None  # (an empty tensor's address is null, which reads as missing)
-    if segments < 1 or segments > _MAX_SEGMENTS or schedule[3].numel() != segments + 1 or max(length, key_slots) > _MAX_COUNT:
+    if segments < 1 or segments > _MAX_SEGMENTS or schedule[3].numel() != segments + 1:
+        return None
+    if max(length, key_slots) > _MAX_COUNT or batch * max(length, key_slots) >= 2**31:
         return None
     a = _native.PlanArgs()
     a.query_indices, a.key_indices, a.cu_queries, a.cu_keys = (t.data_ptr() for t in schedule)

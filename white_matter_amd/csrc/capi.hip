@@ -214,6 +214,10 @@ int check_feedback_meta(const wmx_feedback_meta_args* a) {
 int check_plan(const wmx_plan_args* a, bool fill) {
   if (!a) return fail(WMX_E_INVALID, "args is NULL");
   if (a->batch < 1 || a->q_len < 1 || a->k_len < 1) return fail(WMX_E_INVALID, "plans need a nonempty batch, queries and keys");
+  // the scans count up to three numbers of a row in one word, 21 bits each
+  const int64_t longest = a->q_len > a->k_len ? a->q_len : a->k_len, limit = 1 << 21;
+  if (longest >= limit || a->batch * longest > INT32_MAX)
+    return fail(WMX_E_UNSUPPORTED, "plans take fewer than 2^21 queries and keys a row, and 2^31 in all");
   if (a->query_stride < 1) return fail(WMX_E_INVALID, "query_stride must be >= 1");
   if (a->key_tile != 64 && a->key_tile != 128) return fail(WMX_E_INVALID, "key_tile must be 64 or 128");
   if (a->fused_rows < 0 || a->fused_rows > 128) return fail(WMX_E_INVALID, "fused_rows must be in [0, 128]");
@@ -233,6 +237,8 @@ int check_plan(const wmx_plan_args* a, bool fill) {
   if (!fill) return WMX_OK;
   if (a->total_segments < 1 || a->total_segments >= 1 << 20 || a->num_q_units < 0 || a->num_k_units < 0 || a->num_f_units < 0)
     return fail(WMX_E_INVALID, "invalid plan sizes");
+  if (a->num_q_units >= limit || a->num_k_units >= limit || a->num_f_units >= limit)
+    return fail(WMX_E_UNSUPPORTED, "plans take fewer than 2^21 units a list");
   const bool own = a->out_query_indices && a->out_key_indices && a->out_cu_queries && a->out_cu_keys;
   const bool none = !a->out_query_indices && !a->out_key_indices && !a->out_cu_queries && !a->out_cu_keys;
   if (!own && (a->q_seg || !none || a->total_segments != a->num_segments))
