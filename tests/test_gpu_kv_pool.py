@@ -249,9 +249,9 @@ def test_router_logits_match_fp32_product(rows, inputs, logits):
 @pytest.mark.parametrize(("sources", "hidden", "channels", "stride"), [(5, 64, 3, 1), (9, 128, 4, 2)])
 def test_producer_training_form_gradients(sources, hidden, channels, stride):
     """Under autograd projection_inputs runs the HIP forward (the same bits as
-    without autograd) and the backward differentiates the recomputed eager
-    steps: gradients of every input against float64 autograd through the
-    oracle (bf16 rounding points as casts, which pass gradients through)."""
+    without autograd) and the backward the HIP kernels: gradients of every input
+    against float64 autograd through the oracle (bf16 rounding points as casts,
+    which pass gradients through)."""
     inputs = _producer_inputs(2, 4, sources, hidden, channels, 40 + sources, torch.float32, torch.float32,
                               stride=stride)
     stacked, pre_mix, router, gain = inputs
@@ -290,14 +290,21 @@ def test_producer_training_form_gradients(sources, hidden, channels, stride):
         (1, 5, 16, 136, 16, 1, torch.float32, torch.float32),  # the most channels and logits
         (3, 23, 9, 2048, 4, 2, torch.float32, torch.bfloat16),  # the widest rows
         (1, 70, 64, 1032, 2, 3, torch.bfloat16, torch.float32),  # just past 1024 elements per thread's first share
+        # 7 tokens a source workgroup, one in the last; more 128-token blocks than context workgroups in z
+        (2, 515, 25, 512, 4, 1, torch.float32, torch.bfloat16),
+        (1, 2401, 25, 64, 8, 2, torch.bfloat16, torch.float32),  # 16 tokens a source workgroup, one in the last
+        (1, 37, 11, 1032, 12, 1, torch.float32, torch.float32),  # more than 8 channels, rows past 1024
+        (2, 9, 16, 2048, 16, 1, torch.bfloat16, torch.bfloat16),  # the most of channels, logits and width
     ],
 )
 def test_producer_backward_kernels(batch, tokens, sources, hidden, channels, stride, src_dtype, weight_dtype):
     """The backward kernels against float64 autograd of the oracle at the edges
     of their tiles. The bound: the eager steps they replace round the
     mixtures', the logits' and the premixed rows' gradients to bf16 too, so the
-    kernels' error may not exceed the eager steps' own by more than a tenth
-    (plus one bf16 rounding of a result, 2^-9)."""
+    kernels' error may not exceed the eager steps' own by more than a tenth, plus
+    2^-12: the mixtures are sums in another order, and where fewer than one in a
+    hundred round the other way (a bf16 step, 2^-8 of it at most, 0.6 times that on
+    average), a result moves by sqrt(0.01) * 0.6 * 2^-8."""
     stacked, pre_mix, router, gain = _producer_inputs(
         batch, tokens, sources, hidden, channels, 70 + sources, src_dtype, weight_dtype, stride=stride
     )
@@ -329,7 +336,7 @@ def test_producer_backward_kernels(batch, tokens, sources, hidden, channels, str
         scale = r.norm().clamp_min(1e-30)
         ours, theirs = ((t.double().cpu() - r).norm() / scale for t in (g, e))
         print(f"input {n}: kernels {ours:.2e} eager {theirs:.2e}", flush=True)
-        assert ours <= 1.1 * theirs + 2**-9, f"input {n}: rel-L2 {ours:.3e}, the eager steps' {theirs:.3e}"
+        assert ours <= 1.1 * theirs + 2**-12, f"input {n}: rel-L2 {ours:.3e}, the eager steps' {theirs:.3e}"
 
 
 def test_producer_batched_gradients():
