@@ -15,9 +15,9 @@
 //   reduce  - the sums over tokens of the small gradients, in a fixed order.
 // All of them stream: the sources are read once, p once by mix and its read
 // half once by weight, dm once per group of sources. As torch operations on the
-// recomputed steps the backward took some 150 launches, each over every
-// source in fp32. 1,024 tokens, 25 sources of 1,024, 8 channels, both sides:
-// 2.9 ms as torch operations; here see launch_kv_mix_bwd.
+// recomputed steps the backward took 134 launches, most over every source in
+// fp32. 1,024 tokens, 25 sources of 1,024, 8 channels, both sides: 2.8 ms as
+// torch operations, 0.31 ms here (see launch_kv_mix_bwd).
 #include "lds_tiles.h"
 #include "wmx_kernels.h"
 
@@ -101,8 +101,8 @@ __device__ __forceinline__ float wave_sums(float (&v)[N], int lane) {
   return x;
 }
 
-// EPT consecutive elements (2 or 4) of a bf16 row as fp32.
-template <int EPT>
+// EPT consecutive elements of a bf16 row, as words and as fp32.
+constexpr int EPT = 4;
 __device__ __forceinline__ void unpack(const uint32_t (&w)[EPT / 2], float (&v)[EPT]) {
 #pragma unroll
   for (int i = 0; i < EPT / 2; ++i) {
@@ -110,15 +110,10 @@ __device__ __forceinline__ void unpack(const uint32_t (&w)[EPT / 2], float (&v)[
     v[2 * i + 1] = bf16_hi(w[i]);
   }
 }
-template <int EPT>
 __device__ __forceinline__ void load_words(const bf16* p, uint32_t (&w)[EPT / 2]) {
-  if constexpr (EPT == 4) {
-    const u32x2 x = load8b(p);
-    w[0] = x[0];
-    w[1] = x[1];
-  } else {
-    w[0] = *reinterpret_cast<const uint32_t*>(p);
-  }
+  const u32x2 x = load8b(p);
+  w[0] = x[0];
+  w[1] = x[1];
 }
 
 // mix: workgroup (kMixRows tokens, side) of NT threads; thread t holds elements
@@ -130,7 +125,7 @@ __device__ __forceinline__ void load_words(const bf16* p, uint32_t (&w)[EPT / 2]
 // rows) of dz = dm . p^T, 16x16x32 MFMA blocks of 16 sources whose k-steps are
 // dealt over the waves; B operands come from the token's p rows, which the
 // first half has just read (64 consecutive bytes per row and k-step).
-template <int NT, int EPT, int CM>
+template <int NT, int CM>
 __global__ __launch_bounds__(NT, NT == 256 && CM == 8 ? 2 : NT / 256) void mix_bwd_kernel(const wmx_kv_mix_bwd_args a) {
   constexpr int NW = NT / 64;
   constexpr int LDK = NT * EPT + 8;
@@ -158,8 +153,8 @@ __global__ __launch_bounds__(NT, NT == 256 && CM == 8 ? 2 : NT / 256) void mix_b
     const int64_t at = (int64_t)min(c, C - 1) * H;
     if (a.weight_dtype == WMX_DTYPE_BF16) {
       uint32_t w[EPT / 2];
-      load_words<EPT>(((const bf16*)a.gain[side] + at) + d, w);
-      unpack<EPT>(w, gain[c]);
+      load_words(((const bf16*)a.gain[side] + at) + d, w);
+      unpack(w, gain[c]);
     } else {
 #pragma unroll
       for (int e = 0; e < EPT; ++e) gain[c][e] = (((const float*)a.gain[side]) + at)[d + e];
@@ -172,7 +167,7 @@ __global__ __launch_bounds__(NT, NT == 256 && CM == 8 ? 2 : NT / 256) void mix_b
   uint32_t pw[kBatch][EPT / 2];
   auto load_rows = [&](const bf16* p, int s0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) load_words<EPT>((p + (int64_t)min(s0 + u, S - 1) * H) + d, pw[u]);
+    for (int u = 0; u < kBatch; ++u) load_words((p + (int64_t)min(s0 + u, S - 1) * H) + d, pw[u]);
   };
 #pragma unroll 1
   for (int64_t r = r0; r < r1; ++r) {
@@ -188,7 +183,7 @@ __global__ __launch_bounds__(NT, NT == 256 && CM == 8 ? 2 : NT / 256) void mix_b
     const int64_t gstep = L.rows * H;
 #pragma unroll
     for (int c = 0; c < CM; ++c) {
-      load_words<EPT>((grow + min(c, C - 1) * gstep) + d, g[c]);
+      load_words((grow + min(c, C - 1) * gstep) + d, g[c]);
 #pragma unroll
       for (int i = 0; i < EPT / 2; ++i) g[c][i] = in ? g[c][i] : 0u;
     }
@@ -210,7 +205,7 @@ __global__ __launch_bounds__(NT, NT == 256 && CM == 8 ? 2 : NT / 256) void mix_b
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) {
         float pv[EPT];
-        unpack<EPT>(now[u], pv);
+        unpack(now[u], pv);
 #pragma unroll
         for (int c0 = 0; c0 < CM; c0 += 4) {
           const f32x4 al = *reinterpret_cast<const f32x4*>(z_lds + (s0 + u) * CM + c0);
@@ -227,7 +222,7 @@ __global__ __launch_bounds__(NT, NT == 256 && CM == 8 ? 2 : NT / 256) void mix_b
     for (int c = 0; c < CM; ++c) {
       float ss = 0.f, um = 0.f, gv[EPT];
       __builtin_amdgcn_sched_barrier(0);
-      unpack<EPT>(g[c], gv);
+      unpack(g[c], gv);
 #pragma unroll
       for (int e = 0; e < EPT; ++e) {
         m[c][e] = in ? round_bf16(m[c][e]) : 0.f;
@@ -251,7 +246,7 @@ __global__ __launch_bounds__(NT, NT == 256 && CM == 8 ? 2 : NT / 256) void mix_b
       }
       const float minv = 1.f / sqrtf(ss * rh + a.mix_eps);
       const float k = um * rh * minv * minv * minv;
-      unpack<EPT>(g[c], gv);
+      unpack(g[c], gv);
 #pragma unroll
       for (int e = 0; e < EPT; ++e) {
         dgain[c][e] = fmaf(gv[e], m[c][e] * minv, dgain[c][e]);
@@ -393,13 +388,14 @@ __global__ __launch_bounds__(256) void context_bwd_kernel(const wmx_kv_mix_bwd_a
 // holds elements 1024 v + 4 t + [0, 4). A token's channel rows dm are read once
 // for G sources, from the L2 of the XCD that runs the block's groups one after
 // another. Bound by latency too: with five sources per workgroup (fewer reads of
-// dm, 253 registers) it took 146-159 us, with four 139, with two 88, with one
+// dm, 253 registers) it took 146-159 us, with four 139, with two 83-88, with one
 // 111-120; the barrier of a token waits for LDS only, so its stores fly on.
-template <int VPT, int G, int CM, bool SRC_BF16>
+template <int VPT, int CM, bool SRC_BF16>
 __global__ __launch_bounds__(256, VPT * CM <= 8 ? 2 : 1) void sources_bwd_kernel(const wmx_kv_mix_bwd_args a) {
+  constexpr int G = kGroup, NS = 2 * G;
   static_assert(G == 2, "a channel's logits of the group are one vector read");
   __shared__ __attribute__((aligned(16))) float z_lds[kSourceRows][2][CM * G];
-  __shared__ float red[2][4][16];
+  __shared__ float red[2][4][NS];
   const BwdLayout L(a);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int H = a.hidden, S = a.num_sources, C = a.channels;
@@ -416,7 +412,7 @@ __global__ __launch_bounds__(256, VPT * CM <= 8 ? 2 : 1) void sources_bwd_kernel
   const int nrows = (int)min(L.source_rows, L.rows - r0);
   for (int i = tid; i < nrows * 2 * CM * G; i += 256) {
     const int g = i % G, c = i / G % CM, side = i / (G * CM) % 2, rr = i / (G * CM * 2);
-    const bool in = g < G && s0 + g < S && c < C;
+    const bool in = s0 + g < S && c < C;
     z_lds[rr][side][c * G + g] = in ? (float)((const bf16*)a.alpha[side])[(r0 + rr) * a.alpha_stride + c * S + s0 + g] : 0.f;
   }
   // sources and channels past the last repeat it (with zero logits), elements
@@ -531,21 +527,18 @@ __global__ __launch_bounds__(256, VPT * CM <= 8 ? 2 : 1) void sources_bwd_kernel
         }
       }
     // the norm's backward: dx = inv dy - x inv^3 mean(dy x), dy = sum of pre dp
-    constexpr int NS = 2 * G;
     float sums[NS];
 #pragma unroll
-    for (int g = 0; g < NS / 2; ++g) {
+    for (int g = 0; g < G; ++g) {
       float ss = 0.f, yx = 0.f;
-      if (g < G) {
 #pragma unroll
-        for (int v = 0; v < VPT; ++v)
+      for (int v = 0; v < VPT; ++v)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float dy = pre[0][g][v][e] * dp[0][g][v][e] + pre[1][g][v][e] * dp[1][g][v][e];
-            ss = fmaf(x[g][v][e], x[g][v][e], ss);
-            yx = fmaf(dy, x[g][v][e], yx);
-          }
-      }
+        for (int e = 0; e < 4; ++e) {
+          const float dy = pre[0][g][v][e] * dp[0][g][v][e] + pre[1][g][v][e] * dp[1][g][v][e];
+          ss = fmaf(x[g][v][e], x[g][v][e], ss);
+          yx = fmaf(dy, x[g][v][e], yx);
+        }
       sums[2 * g] = ss;
       sums[2 * g + 1] = yx;
     }
@@ -554,7 +547,7 @@ __global__ __launch_bounds__(256, VPT * CM <= 8 ? 2 : 1) void sources_bwd_kernel
     lds_barrier();  // (the other buffer is read again two tokens on, past the next barrier)
 #pragma unroll
     for (int g = 0; g < G; ++g) {
-      const float(&s)[4][16] = red[rr & 1];
+      const float(&s)[4][NS] = red[rr & 1];
       const float ss = s[0][2 * g] + s[1][2 * g] + s[2][2 * g] + s[3][2 * g];
       const float yx = s[0][2 * g + 1] + s[1][2 * g + 1] + s[2][2 * g + 1] + s[3][2 * g + 1];
       const float inv = 1.f / sqrtf(ss * rh + a.eps);
@@ -590,8 +583,8 @@ __global__ __launch_bounds__(256, VPT * CM <= 8 ? 2 : 1) void sources_bwd_kernel
               f32x4{dpre[side][g][v][0], dpre[side][g][v][1], dpre[side][g][v][2], dpre[side][g][v][3]};
 }
 
-// weight: dW = dz^T . p for 128 columns of the router's view, all logits, over
-// every token: tiles of 64 tokens of p (its columns in place) and of dz, both
+// weight: dW = dz^T . p for 128 columns of the router's view, all logits, one
+// workgroup over every token: tiles of 64 tokens of p (its columns in place) and of dz, both
 // read transposed; wave w owns columns 32 w .. 32 w + 31. Two buffers, the next
 // tiles stream in during the products.
 template <int NB>
@@ -708,14 +701,14 @@ __global__ __launch_bounds__(1024) void reduce_bwd_kernel(const wmx_kv_mix_bwd_a
 
 template <int NT, int CM>
 void launch_mix(const wmx_kv_mix_bwd_args& a, const BwdLayout& L, hipStream_t stream) {
-  hipLaunchKernelGGL((mix_bwd_kernel<NT, 4, CM>), dim3((unsigned)L.mix_blocks, 2), dim3(NT), 0, stream, a);
+  hipLaunchKernelGGL((mix_bwd_kernel<NT, CM>), dim3((unsigned)L.mix_blocks, 2), dim3(NT), 0, stream, a);
 }
 
 template <int VPT, int CM>
 void launch_sources(const wmx_kv_mix_bwd_args& a, const BwdLayout& L, hipStream_t stream) {
   const dim3 grid((unsigned)((L.source_blocks + 7) / 8 * 8 * L.groups));
-  if (a.source_dtype == WMX_DTYPE_BF16) hipLaunchKernelGGL((sources_bwd_kernel<VPT, kGroup, CM, true>), grid, dim3(256), 0, stream, a);
-  else hipLaunchKernelGGL((sources_bwd_kernel<VPT, kGroup, CM, false>), grid, dim3(256), 0, stream, a);
+  if (a.source_dtype == WMX_DTYPE_BF16) hipLaunchKernelGGL((sources_bwd_kernel<VPT, CM, true>), grid, dim3(256), 0, stream, a);
+  else hipLaunchKernelGGL((sources_bwd_kernel<VPT, CM, false>), grid, dim3(256), 0, stream, a);
 }
 
 template <int NB>
@@ -728,8 +721,8 @@ void launch_weight(const wmx_kv_mix_bwd_args& a, const BwdLayout& L, hipStream_t
 int64_t kv_mix_bwd_workspace_size(const wmx_kv_mix_bwd_args& a) { return BwdLayout(a).bytes; }
 
 // Measured at 1,024 tokens, 25 sources of 1,024, 8 channels: mix 92 us, context
-// 37, sources 88, weight 38, reduce 19 us, after 38 us for the premixed rows
-// again; forward and backward with the key transform 3.0 ms -> 0.5 ms.
+// 37, sources 83-88, weight 38, reduce 17-19 us, after 38 us for the premixed rows
+// again; forward and backward with the key transform 3.0 ms -> 0.57-0.66 ms.
 int launch_kv_mix_bwd(const wmx_kv_mix_bwd_args& a, hipStream_t stream) {
   const BwdLayout L(a);
   if (L.mix_blocks > INT32_MAX) return WMX_E_UNSUPPORTED;
