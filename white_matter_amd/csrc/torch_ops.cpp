@@ -1012,7 +1012,9 @@ void rope_rows(const Tensor& cos, const Tensor& sin, const Tensor& weight, const
   c10::OptionalDeviceGuard guard(x.device());
   auto step = [](const Tensor& t, int d) { return t.size(d) > 1 ? t.stride(d) : 0; };
   auto rows = [&](const Tensor& t) {
-    const Tensor e = t.to(at::kFloat).expand(want);
+    Tensor e = t;  // (a host microsecond each, so only where they change something)
+    if (e.scalar_type() != at::kFloat) e = e.to(at::kFloat);
+    if (e.sizes() != c10::IntArrayRef(want)) e = e.expand(want);
     const bool ok = e.stride(-1) == 1 && reinterpret_cast<uintptr_t>(e.data_ptr()) % 16 == 0 && step(e, 0) % 4 == 0 &&
                     step(e, 1) % 4 == 0;
     return ok ? e : dense16(e);

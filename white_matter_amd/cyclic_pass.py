@@ -264,7 +264,7 @@ class FeedbackModel:
             and not (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != self.dtype)
             and all(
                 t.dtype in _ROPE_DTYPES and t.ndim == 3
-                and all(n in (1, m) for n, m in zip(t.shape, (*x.shape[:2], c.head_dim)))
+                and all(n == 1 or n == m for n, m in zip(t.shape, (*x.shape[:2], c.head_dim)))
                 for t in rope
             )
         )
